@@ -953,17 +953,69 @@ class _RowOffsets:
 
 def emit_reduction(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
     if k.two_pass:
-        return emit_streamed(k, cfg)
+        wide = resident_geometry(k)
+        return emit_streamed(k, cfg) if wide is None else emit_persistent(k, cfg, wide)
     return emit_persistent(k, cfg)
 
 
-def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
+#: resident streamed rows: one workgroup of this many lanes per row, and at
+#: most this many register elements per lane over the row's column operands
+RESIDENT = {"lanes": 1024, "elements": 64}
+
+
+def resident_geometry(k: ReductionKernel) -> dict | None:
+    """Geometry of a streamed row that fits one workgroup's registers, or
+    ``None`` for the chunk loop (``emit_streamed``).
+
+    A streamed row is read once per pass by the chunk loop, two bytes at a
+    time when its length is odd: softmax over 512 rows of 50257 fp16 took
+    146 us, bound by per-element loads and the online recurrence's serial
+    chain of exponentials. 1024 lanes hold up to 65536 elements (64 fp32
+    registers each, half of the 128 a full workgroup leaves a lane), so such a
+    row is read once and reduced like a persistent one: that call, its input
+    copy included, went from 171 to 53 us.
+
+    A row that does not start on a pack boundary (an odd row length) is
+    covered by the packs of its buffer's own 16-byte grid: ``shift`` elements
+    of the first pack belong to the row before. The first and last pack move
+    per element. That needs every column operand at unit stride and at the
+    same distance from its grid. The lower limit is two packs per lane: a
+    shorter row leaves half of the lanes idle."""
+    col_args = [a for a in k.inputs if a.index.varies_along("col")]
+    n_loaded = len(col_args)
+    col_args += [a for a in k.outputs if a.value.name not in k.row_outputs]
+    if not n_loaded or any(itemsize(a.dtype) not in (2, 4) or compute_type(a.dtype) != "float"
+                           for a in col_args):
+        return None
+    if any(t not in ("float", "bool") for t in _step_types(k).values()):
+        return None
+    C = k.reduce_numel
+    V = _vec_width([a.dtype for a in col_args])
+    if any(axis_terms(a.index, "col") != ((C, 1, 1),) for a in col_args):
+        return None
+    starts = {(tuple((t[0], t[1], t[2] % V) for t in axis_terms(a.index, "row") if t[2] % V),
+               a.index.base % V) for a in col_args}
+    if len(starts) != 1:
+        return None
+    shifted = starts != {((), 0)} or C % V != 0
+    G = RESIDENT["lanes"]
+    nvec = -(-C // V) + (1 if shifted else 0)  # a shifted row can touch one pack more
+    K = -(-nvec // G)
+    if nvec < 2 * G or K * V * n_loaded > RESIDENT["elements"]:
+        return None
+    return {"G": G, "K": K, "rows_per_wg": 1, "block": G, "V": V,
+            "shift": col_args[0] if shifted else None}
+
+
+def emit_persistent(k: ReductionKernel, cfg: Config,
+                    wide: dict | None = None) -> tuple[str, LaunchSpec]:
     R, C = k.n_rows, k.reduce_numel
     it = index_type(k)
-    V = _choose_reduction_vec(k)
-    geo = reduction_geometry(R, C, V)
+    V = _choose_reduction_vec(k) if wide is None else wide["V"]
+    geo = reduction_geometry(R, C, V) if wide is None else wide
     G, K, RPW, WG = geo["G"], geo["K"], geo["rows_per_wg"], geo["block"]
-    exact = C == G * K * V
+    shift = geo.get("shift")
+    exact = C == G * K * V and shift is None
     offs = _RowOffsets(k, it)
     col_slots = [i for i, a in enumerate(k.inputs) if a.index.varies_along("col")]
     vector = varies_by_column(k)
@@ -973,8 +1025,8 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
     L: list[str] = []
     L.append(f"extern \"C\" __global__ void __launch_bounds__({WG}) "
              f"KERNEL({', '.join(_params(k))}) {{")
-    L.append(f"  // persistent: {R} rows of {C}; {G} lanes x {K} packs x {V} per row, "
-             f"{RPW} rows per workgroup")
+    L.append(f"  // {'persistent' if wide is None else 'streamed, resident'}: {R} rows of {C}; "
+             f"{G} lanes x {K} packs x {V} per row, {RPW} rows per workgroup")
     L.append(f"  constexpr {it} R = ({it}){R};")
     L.append(f"  constexpr {it} C = ({it}){C};")
     L.append(f"  constexpr int G = {G}, K = {K}, V = {V};")
@@ -988,7 +1040,23 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
     L.append(f"  const {it} lane = threadIdx.x % G;")
     if R % RPW != 0:
         L.append("  if (row >= R) return;")
-    if not exact:
+    # first column of pack p; before the row (it wraps) for the first pack of
+    # a shifted row
+    c0 = f"(({it})p * G + lane) * V"
+    if shift is not None:
+        L.append(f"  const {it} shift = {offs.row(shift)} % ({it})V;")
+        c0 += " - shift"
+        # valid: some column of the pack lies in the row; whole: all of them.
+        # Both are constants for every pack but the first and the last ones.
+        L.append("  bool valid[K], whole[K];")
+        L.append("#pragma unroll")
+        L.append("  for (int p = 0; p < K; ++p) {")
+        L.append(f"    const {it} g0 = (({it})p * G + lane) * V;")
+        L.append(f"    const bool inside = ({it})(p + 1) * G * V <= C;")
+        L.append("    valid[p] = inside || g0 < shift + C;")
+        L.append("    whole[p] = (p > 0 || g0 >= shift) && (inside || g0 + V <= shift + C);")
+        L.append("  }")
+    elif not exact:
         L.append("  bool valid[K];")
         L.append("#pragma unroll")
         L.append(f"  for (int p = 0; p < K; ++p) valid[p] = (({it})p * G + lane) * V < C;")
@@ -1004,15 +1072,21 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
         L.append(f"  {{ const {it} rb = {offs.row(a)};")
         L.append("#pragma unroll")
         L.append("    for (int p = 0; p < K; ++p) {")
-        L.append(f"      const {it} c0 = (({it})p * G + lane) * V;")
-        guard = "" if exact else "if (valid[p]) "
+        L.append(f"      const {it} c0 = {c0};")
         if not exact:
             L.append("      if (!valid[p]) {")
             L.append("#pragma unroll")
             L.append(f"        for (int j = 0; j < V; ++j) v{i}[p][j] = ({ct})0;")
             L.append("        continue;")
             L.append("      }")
-        if acc.mode == "affine" and acc.aligned:
+        if shift is not None:
+            L.append(f"      if (whole[p]) mlc::load_pack<V>(v{i}[p], in{i} + ({it})(rb + c0));")
+            L.append("      else {")
+            L.append("#pragma unroll")
+            L.append(f"        for (int j = 0; j < V; ++j) v{i}[p][j] = ({it})(c0 + j) < C ? "
+                     f"mlc::ld(in{i} + ({it})(rb + c0 + j)) : ({ct})0;")
+            L.append("      }")
+        elif acc.mode == "affine" and acc.aligned:
             L.append(f"      mlc::load_pack<V>(v{i}[p], in{i} + rb + {offs.col(a, 'c0')});")
         elif acc.mode == "affine":
             L.append(f"      const {it} o = rb + {offs.col(a, 'c0')};")
@@ -1023,7 +1097,6 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
             L.append(f"      for (int j = 0; j < V; ++j) v{i}[p][j] = mlc::ld(in{i} + rb + {offs.col(a, '(c0 + (' + it + ')j)')});")
         L.append("    }")
         L.append("  }")
-        del guard
 
     def ref_elem(slot):
         if slot in col_slots:
@@ -1045,7 +1118,7 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
 
     nonpos = nonpositive_args(k)
     half_slots, defs, to_fp16 = half_inputs(k), bind_defs(k), fp16_rounded(k)
-    vt = value_types_of(k)
+    vt = value_types_of(k, frozenset() if wide is None else online_names(plan_passes(k)))
     narrow = narrow_values(vt)
     elem_r = _NonPosExpRenderer(ref_elem, temp_elem, nonpos, half_slots, defs, to_fp16,
                                 fast_softmax_exps(k, nonpos) - narrow, vt)
@@ -1097,6 +1170,13 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
             L.append("    for (int p = 0; p < K; ++p) {")
             if not exact:
                 L.append("      if (!valid[p]) continue;")
+            if shift is not None:
+                L.append("      if (!whole[p]) {")
+                L.append("#pragma unroll")
+                L.append(f"        for (int j = 0; j < V; ++j) if (({it})({c0} + j) < C) "
+                         f"acc = {op}::f(acc, ({t})({code}));")
+                L.append("        continue;")
+                L.append("      }")
             L.append("#pragma unroll")
             L.append(f"      for (int j = 0; j < V; ++j) acc = {op}::f(acc, ({t})({code}));")
             L.append("    }")
@@ -1109,7 +1189,8 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
             L.append("    for (int p = 0; p < K; ++p) {")
             if not exact:
                 L.append("      if (!valid[p]) continue;")
-            L.append(f"      for (int j = 0; j < V; ++j) acc = {op}::f(acc, x);")
+            guard = "" if shift is None else f"if (({it})({c0} + j) < C) "
+            L.append(f"      for (int j = 0; j < V; ++j) {guard}acc = {op}::f(acc, x);")
             L.append("    }")
         slot = f"lds_{s.name}" if G > WAVE else "nullptr"
         L.append(f"    {s.name} = {_reduced(s, vt, f'mlc::row_reduce<G, {op}>(acc, ({t}*){slot})')};")
@@ -1130,7 +1211,7 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
         L.append("    for (int p = 0; p < K; ++p) {")
         if not exact:
             L.append("      if (!valid[p]) continue;")
-        L.append(f"      const {it} c0 = (({it})p * G + lane) * V;")
+        L.append(f"      const {it} c0 = {c0};")
         half_out = a.dtype == torch.float16
         if _expr_varies(e, col_slots, vector):
             code, _ = elem_r.store(e, half_out)
@@ -1139,7 +1220,14 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
         L.append(f"      {ot} o[V];")
         L.append("#pragma unroll")
         L.append(f"      for (int j = 0; j < V; ++j) o[j] = {code};")
-        if acc.mode == "affine" and acc.aligned:
+        if shift is not None:
+            L.append(f"      if (whole[p]) mlc::store_pack<V>(out{i} + ({it})(rb + c0), o);")
+            L.append("      else {")
+            L.append("#pragma unroll")
+            L.append(f"        for (int j = 0; j < V; ++j) if (({it})(c0 + j) < C) "
+                     f"mlc::st(out{i} + ({it})(rb + c0 + j), o[j]);")
+            L.append("      }")
+        elif acc.mode == "affine" and acc.aligned:
             L.append(f"      mlc::store_pack<V>(out{i} + rb + {offs.col(a, 'c0')}, o);")
         else:
             L.append("#pragma unroll")
@@ -1158,7 +1246,9 @@ def emit_persistent(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
     L.append("}")
 
     grid = -(-R // RPW)
-    spec = LaunchSpec("", grid, WG, lds, {"kind": "reduction", "mode": "persistent", "vec": V,
+    mode = "persistent" if wide is None else "streamed"
+    spec = LaunchSpec("", grid, WG, lds, {"kind": "reduction", "mode": mode, "vec": V,
+                                          "resident": True,
                                           "lanes_per_row": G, "packs": K, "rows_per_wg": RPW,
                                           "rows": R, "cols": C})
     return "\n".join(L), spec
@@ -1350,6 +1440,12 @@ def _expr_varies(e: Expr, col_slots, vector) -> bool:
 STREAM_BLOCK = 256
 
 
+def online_names(passes) -> frozenset[str]:
+    """The max and sum steps a pass plan computes with the online recurrence."""
+    return frozenset(n for p in passes if p.online_softmax is not None
+                     for n in (p.online_softmax.max_step.name, p.online_softmax.sum_step.name))
+
+
 def emit_streamed(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
     """One row per workgroup; each pass of the reduction schedule streams the
     row from HBM in chunks of ``STREAM_BLOCK * V`` elements."""
@@ -1404,10 +1500,7 @@ def emit_streamed(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
 
     nonpos = nonpositive_args(k)
     half_slots, defs, to_fp16 = half_inputs(k), bind_defs(k), fp16_rounded(k)
-    online_names = frozenset(n for p in passes if p.online_softmax is not None
-                             for n in (p.online_softmax.max_step.name,
-                                       p.online_softmax.sum_step.name))
-    vt = value_types_of(k, online_names)
+    vt = value_types_of(k, online_names(passes))
     narrow = narrow_values(vt)
     elem_r = _NonPosExpRenderer(ref_elem, temp_elem, nonpos, half_slots, defs, to_fp16, vtypes=vt)
     scal_r = Renderer(lambda s: (f"v{s}", in_types[s]), temp_scalar, half_slots, defs, to_fp16, vt)
@@ -1546,6 +1639,7 @@ def emit_streamed(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
         L.append("  }")
     L.append("}")
     spec = LaunchSpec("", R, G, lds, {"kind": "reduction", "mode": "streamed", "vec": V,
+                                      "resident": False,
                                       "lanes_per_row": G, "passes": len(passes),
                                       "rows": R, "cols": C})
     return "\n".join([x for x in L if x != ""]), spec
