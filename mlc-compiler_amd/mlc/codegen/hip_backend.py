@@ -1788,21 +1788,35 @@ def generate_module(schedule: Schedule, cfg: Config) -> str:
     return build_module(schedule, cfg).source
 
 
-def build_module(schedule: Schedule, cfg: Config) -> Module:
-    """Source, launch table and per-symbol bodies of ``schedule``'s module.
+def _module(emitted, prelude: str) -> Module:
+    """``(kernel name, (body, spec) or None)`` pairs as one translation unit.
     Identical kernel bodies are emitted once, under a symbol named by the
     body's hash."""
     functions: dict[str, str] = {}
     launches: dict[str, LaunchSpec] = {}
-    for k in schedule.kernels:
-        emitted = emit_kernel(k, cfg)
-        if emitted is None:
+    for name, found in emitted:
+        if found is None:
             continue
-        body, spec = emitted
+        body, spec = found
         digest = hashlib.sha256(body.encode()).hexdigest()[:16]
         symbol = f"mlc_{digest}"
         functions.setdefault(symbol, body.replace("KERNEL(", f"{symbol}(", 1))
         spec.symbol = symbol
-        launches[k.name] = spec
-    parts = [PRELUDE] + [functions[s] for s in sorted(functions)]
+        launches[name] = spec
+    parts = [prelude] + [functions[s] for s in sorted(functions)]
     return Module("\n\n".join(parts) + "\n", launches, functions)
+
+
+def build_module(schedule: Schedule, cfg: Config) -> Module:
+    """Source, launch table and per-symbol bodies of ``schedule``'s module."""
+    return _module(((k.name, emit_kernel(k, cfg)) for k in schedule.kernels), PRELUDE)
+
+
+def build_products(schedule: Schedule) -> Module:
+    """The same for the library calls that run as native matrix products
+    (``hip_gemm``), a module of their own: its text depends on the products'
+    sizes alone, so schedules of one model share its code object."""
+    from .hip_gemm import emit_product
+
+    return _module(((k.name, emit_product(k)) for k in schedule.kernels
+                    if isinstance(k, ExternKernel)), PRELUDE + '#include "mlc_gemm.h"\n')

@@ -1,0 +1,245 @@
+"""Native matrix products for the library calls of a schedule.
+
+``aten.mm``, ``aten.addmm`` and ``aten.bmm`` stay extern kernels of the
+schedule; where a product is small enough that a library GEMM's fixed cost is
+most of its time, the runtime runs one of the two templates of
+``templates/mlc_gemm.h`` in the library call's place (``plan_product`` decides,
+from sizes, strides and types alone). Both accumulate in fp32 and round once
+to the storage type, as the library does; ``addmm``'s bias is added before that
+rounding.
+
+* **tiled** (``gemm_tile``): both operands at unit stride along k, in aligned
+  rows of whole 128-byte pieces -- a linear layer's activations and its
+  ``[N, K]`` weight. Operands go straight from memory into an LDS ring.
+* **staged** (``gemm_staged``): any strides, sizes and alignments, through
+  registers into LDS -- attention's products over strided heads or odd lengths.
+
+Measured in graphs of 24-48 products over 12 weights, fp16, library / tiled:
+16x2048x512 (M x N x K) 3.6 / 2.0 us, 128x768x768 4.6 / 2.3, 128x3072x768
+7.8 / 3.7, 128x768x3072 7.6 / 4.8, 512x768x768 7.2 / 3.7, 1182x768x768
+7.9 / 5.2, 2048x2304x768 16.3 / 12.5, 2048x768x3072 18.8 / 18.3; past 10 GFLOP
+the library wins (4096x2304x768 20.1 / 24.0). fp32: 128x3072x768 15.3 / 7.6,
+128x768x3072 12.0 / 9.7, 1024x768x768 14.1 / 12.4, 1024x2304x768 36.4 / 39.
+"""
+
+from __future__ import annotations
+
+import math
+from dataclasses import dataclass
+
+import torch
+
+from ..ir.graph import Value
+from ..kernels import ExternKernel
+from .hip_backend import STORAGE, LaunchSpec, itemsize
+
+CUS, XCDS = 256, 8
+LDS_BYTES = 160 * 1024
+
+#: tiled form: rows and columns of a workgroup's tile, waves across them, and
+#: the k-splits tried
+TILES = ((16, 16, 1, 1, (1, 2, 4)), (16, 32, 1, 2, (2, 4)), (16, 32, 1, 1, (3,)),
+         (32, 32, 2, 2, (1, 2, 4)), (32, 48, 2, 1, (2, 4)), (32, 64, 2, 2, (1, 2)),
+         (64, 64, 2, 2, (1, 2)), (64, 96, 2, 2, (1, 2)), (64, 128, 2, 4, (1,)),
+         (96, 96, 2, 2, (1,)), (128, 96, 2, 2, (1,)), (128, 128, 2, 4, (1,)),
+         (128, 192, 2, 4, (1,)))
+#: floating-point operations up to which the tiled form is at least the
+#: library's speed (the table above), by element size
+TILED_FLOPS = {2: 10e9, 4: 2.2e9}
+#: widest product measured: a vocabulary head streams its weights, where the
+#: library's larger tiles win
+MAX_COLUMNS = 4096
+
+
+@dataclass(frozen=True)
+class Operand:
+    """A ``[batch, rows, k]`` view of a buffer (strides in elements)."""
+
+    value: Value
+    batch: int
+    row: int
+    k: int
+    base: int
+
+    def aligned(self, elements: int, batches: int) -> bool:
+        """Every row starts on a multiple of ``elements``."""
+        return (self.k == 1 and self.row % elements == 0 and self.base % elements == 0
+                and (batches == 1 or self.batch % elements == 0))
+
+
+@dataclass(frozen=True)
+class Product:
+    """``out[z, m, n] = sum_k a[z, m, k] b[z, n, k] (+ bias[n])``."""
+
+    batches: int
+    M: int
+    N: int
+    K: int
+    a: Operand
+    b: Operand
+    out: Operand      # rows m, k-axis n
+    bias: Value | None
+    form: tuple       # ("tiled", TM, TN, WM, WN, WK, stages) or ("staged", TM, TN)
+
+
+def _operand(v: Value, row_axis: int, k_axis: int) -> Operand:
+    lay = v.layout
+    return Operand(v, lay.strides[0] if len(v.shape) == 3 else 0, lay.strides[row_axis],
+                   lay.strides[k_axis], lay.offset)
+
+
+def tile_cost(M: int, N: int, K: int, batches: int, size: int, tile: tuple) -> float:
+    """Microseconds of the tiled form in one launch, fitted to 1300 timings
+    (median error 6%): a launch and its epilogue, the first load's latency once
+    per round of workgroups, and for the busiest CU's tiles the larger of its
+    LDS reads and its matrix instructions, plus its loads."""
+    TM, TN, WM, WN, WK, stages = tile
+    tiles = batches * -(-M // TM) * -(-N // TN)
+    steps = K * size // 128 // WK
+    ring = min(stages, steps) * WK * (TM + TN) * 128
+    waves = WM * WN * WK
+    together = max(1, min(LDS_BYTES // ring, 16 // waves))
+    per_xcd = -(-tiles // XCDS)
+    per_cu = -(-per_xcd // (CUS // XCDS))
+    rounds = -(-per_xcd // (CUS // XCDS * together))
+    loads = (TM + TN) * K * size
+    reads = (TM * WN + TN * WM) * K * size
+    macs = TM * TN * K * (1 if size == 2 else 8)
+    simds = min(4, waves * min(together, per_cu))
+    return (1.1 + 0.8 * rounds + per_cu * (max(2.95e-6 * reads, 4.33e-7 * macs * 4 / simds)
+                                           + 5.66e-6 * loads + 6e-6 * TM * TN))
+
+
+def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None:
+    """The cheapest tile by ``tile_cost``, with the deepest ring that fits LDS.
+
+    In fp32 a k-split of 4 is kept up to 128 rows, where the library sums k in
+    as many parts: fewer, longer sums would be further from float64 than it
+    is (5.0e-7 relative against 2.5e-7 at K = 768)."""
+    pieces = K * size // 128
+    best = None
+    for TM, TN, WM, WN, splits in TILES:
+        if TM > max(16, 2 * M):
+            continue
+        fewest = 1
+        if size == 4:
+            fewest = (4 if M <= 128 else 2) if TM * TN <= 32 * 48 else 2 if TM * TN <= 64 * 96 else 1
+        for WK in sorted({min(n, pieces) for n in splits}):
+            if pieces % WK or WK < min(fewest, pieces):
+                continue
+            steps = pieces // WK
+            stages = next((n for n in (4, 3, 2)
+                           if min(n, steps) * WK * (TM + TN) * 128 <= LDS_BYTES), None)
+            if stages is None:
+                continue
+            tile = (TM, TN, WM, WN, WK, min(stages, max(2, steps)))
+            cost = tile_cost(M, N, K, batches, size, tile)
+            if best is None or cost < best[0]:
+                best = (cost, tile)
+    return best[1] if best else None
+
+
+#: staged form: operations up to which it is used, and the rows and columns of
+#: its tile
+STAGED_FLOPS = 2e9
+
+
+def plan_product(k: ExternKernel) -> Product | None:
+    """How a library call's product runs natively, or ``None`` to leave it to
+    the library."""
+    node = k.node
+    op = node.op
+    if op not in ("aten.mm.default", "aten.addmm.default", "aten.bmm.default") or node.kwargs:
+        return None
+    args, bias = list(node.args), None
+    if op == "aten.addmm.default":
+        bias, args = args[0], args[1:]
+    if len(args) != 2 or len(node.outputs) != 1 or not all(isinstance(v, Value) for v in args):
+        return None
+    x, w = args
+    out = node.outputs[0]
+    rank = 3 if op == "aten.bmm.default" else 2
+    if any(len(v.shape) != rank for v in (x, w, out)) or len({v.dtype for v in (x, w, out)}) != 1:
+        return None
+    if x.dtype not in (torch.float16, torch.bfloat16, torch.float32):
+        return None
+    M, K, N = x.shape[-2], x.shape[-1], w.shape[-1]
+    batches = x.shape[0] if rank == 3 else 1
+    if w.shape[-2] != K or tuple(out.shape[-2:]) != (M, N) or min(M, N, K, batches) < 1:
+        return None
+    if bias is not None and not (isinstance(bias, Value) and tuple(bias.shape) == (N,)
+                                 and bias.dtype == x.dtype and (N == 1 or bias.layout.strides[0] == 1)):
+        return None
+    operands = [v for v in (x, w, out, bias) if v is not None]
+    if any(v.buffer.numel >= 2 ** 31 or min(v.layout.strides, default=0) < 0 for v in operands):
+        return None
+    a, b, c = _operand(x, -2, -1), _operand(w, -1, -2), _operand(out, -2, -1)
+    if N > 1 and c.k != 1:
+        return None
+    size = itemsize(x.dtype)
+    flops = 2.0 * batches * M * N * K
+    E = 16 // size
+    if (K * size % 128 == 0 and N <= MAX_COLUMNS and flops <= TILED_FLOPS[size]
+            and a.aligned(E, batches) and b.aligned(E, batches)):
+        tile = choose_tile(M, N, K, batches, size)
+        if tile is not None:
+            return Product(batches, M, N, K, a, b, c, bias, ("tiled", *tile))
+    if rank == 3 and flops <= STAGED_FLOPS:
+        return Product(batches, M, N, K, a, b, c, bias, ("staged", *staged_tile(M, N, batches)))
+    return None
+
+
+def staged_tile(M: int, N: int, batches: int) -> tuple[int, int]:
+    """64 x 64, or 32 wide along an axis where 64 leaves half of the chip idle."""
+    TM = TN = 64
+    if batches * -(-M // 64) * -(-N // 64) < CUS:
+        TM = 32
+        if batches * -(-M // 32) * -(-N // 64) < CUS:
+            TN = 32
+    return TM, TN
+
+
+def emit_product(k: ExternKernel) -> tuple[str, LaunchSpec] | None:
+    """Source (with the placeholder name ``KERNEL``) and launch spec of a
+    library call's native product, or ``None``."""
+    p = plan_product(k)
+    if p is None:
+        return None
+    T = STORAGE[p.a.value.dtype]
+    E = 16 // itemsize(p.a.value.dtype)
+    form, TM, TN = p.form[:3]
+    mt, nt = -(-p.M // TM), -(-p.N // TN)
+    tiles = p.batches * mt * nt
+    threads = 64 * math.prod(p.form[3:6]) if form == "tiled" else 256
+    packed = p.N % 4 == 0 and p.out.aligned(4, p.batches)
+    bias = f", const {T}* __restrict__ bias" if p.bias is not None else ""
+    L = [f"extern \"C\" __global__ void __launch_bounds__({threads}) "
+         f"KERNEL(const {T}* __restrict__ a, const {T}* __restrict__ b{bias}, {T}* __restrict__ c) {{",
+         f"  // {form}: {p.batches} x [{p.M} x {p.K}] x [{p.K} x {p.N}], {TM} x {TN} tiles",
+         "  int t;",
+         f"  if (!mlc::tile_index<{tiles}>(t)) return;",
+         f"  const int z = t / {mt * nt}, mt = t % {mt}, nt = t / {mt} % {nt};"]
+    for name, o in (("a", p.a), ("b", p.b), ("c", p.out)):
+        L.append(f"  {name} += (int64_t)z * {o.batch if p.batches > 1 else 0} + {o.base};")
+    L += ["  auto store = [&](int m, int n, mlc::float4v s) {",
+          "    float v[4] = {s[0], s[1], s[2], s[3]};"]
+    if p.bias is not None:
+        L += ["#pragma unroll",
+              f"    for (int i = 0; i < 4; ++i) if (n + i < {p.N}) "
+              f"v[i] += mlc::ld(bias + {p.bias.layout.offset} + n + i);"]
+    L += [f"    mlc::store4<{T}, {p.M}, {p.N}, {p.out.row}, {str(packed).lower()}>(c, m, n, v);",
+          "  };"]
+    if form == "tiled":
+        L.append(f"  mlc::gemm_tile<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.b.row}, "
+                 f"{', '.join(map(str, p.form[1:]))}>(a, b, mt * {TM}, nt * {TN}, store);")
+    else:
+        flags = ", ".join(str(o.aligned(E, p.batches) and p.K % E == 0).lower() for o in (p.a, p.b))
+        L.append(f"  mlc::gemm_staged<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.a.k}, {p.b.row}, {p.b.k}, "
+                 f"{TM}, {TN}, {8 * E}, {flags}>(a, b, mt * {TM}, nt * {TN}, store);")
+    L.append("}")
+    values = [p.a.value, p.b.value, *([p.bias] if p.bias is not None else []), p.out.value]
+    spec = LaunchSpec("", XCDS * -(-tiles // XCDS), threads, 0,
+                      {"kind": "gemm", "form": p.form, "buffers": [v.buffer.name for v in values],
+                       "dtypes": [v.buffer.dtype for v in values],
+                       "numels": [v.buffer.numel for v in values]})
+    return "\n".join(L), spec

@@ -23,7 +23,8 @@ when the op has an ``.out`` overload taking exactly its arguments plus
 ``out`` (read off the schemas, never by calling it) the result is written
 straight into its buffer; otherwise the op is called and its result copied.
 The HIP runtime may claim an op with a native kernel instead (``NativeCall``:
-the bounds-checked embedding gather).
+the bounds-checked embedding gather; ``ProductCall``: a matrix product small
+enough to beat the library).
 
 Behaviour kept from the reference runtime (``mlc/runtime/executor.py:41-474``):
 the input checks and their messages, output aliasing, the eager mode, three
@@ -129,12 +130,25 @@ class NativeCall:
         self.module.run_bound(self.bound)
 
 
+@dataclass
+class ProductCall:
+    """A library GEMM's product run by a native kernel of the runtime: the
+    same operation at the same precision, its sum over k in another order."""
+
+    module: Any
+    bound: Any
+
+    def run(self) -> None:
+        self.module.run_bound(self.bound)
+
+
 def bind_extern(k: ExternKernel, buffers: dict[str, torch.Tensor], module=None):
     """Resolve a library call against the buffer table without running it."""
-    claim = getattr(module, "bind_native_extern", None)
-    bound = claim(k, buffers) if claim is not None else None
-    if bound is not None:
-        return NativeCall(module, bound)
+    for claim, call in (("bind_native_extern", NativeCall), ("bind_product", ProductCall)):
+        bind = getattr(module, claim, None)
+        bound = bind(k, buffers) if bind is not None else None
+        if bound is not None:
+            return call(module, bound)
     node = k.node
     target = node.meta.get("target")
     if target is None:

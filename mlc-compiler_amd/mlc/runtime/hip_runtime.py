@@ -31,7 +31,7 @@ from dataclasses import dataclass
 
 import torch
 
-from ..codegen.hip_backend import LaunchSpec, build_module
+from ..codegen.hip_backend import LaunchSpec, build_module, build_products
 from ..config import Config
 from ..kernels import ExternKernel, Kernel, Schedule
 from . import native
@@ -80,21 +80,20 @@ class HipRuntime:
         #: the generated HIP module text (``TritonRuntime.source``)
         self.source: str = self.module.source
         self.launch_table: dict[str, LaunchSpec] = self.module.launches
-        self.path, self.code_object_path = native.compile_code_object(self.source)
-        image = self.code_object_path.read_bytes()
+        #: library products that run natively, by kernel name; their module
+        #: is loaded beside the generated one when there are any
+        products = build_products(schedule)
+        self.product_table: dict[str, LaunchSpec] = products.launches
+        objects = native.compile_code_objects(
+            [self.source] + ([products.source] if products.launches else []))
+        self.path, self.code_object_path = objects[0]
 
         self._ctx = ctypes.c_void_p()
         native.check(self.lib.mlc_ctx_create(self.index, ctypes.byref(self._ctx)), "mlc_ctx_create")
-        self._mod = ctypes.c_void_p()
-        buf = ctypes.create_string_buffer(image, len(image))
-        native.check(self.lib.mlc_module_load(self._ctx, buf, len(image), ctypes.byref(self._mod)),
-                     "mlc_module_load")
+        self._mods: list[ctypes.c_void_p] = []
         self.functions: dict[str, int] = {}
-        for symbol in sorted({s.symbol for s in self.launch_table.values()}):
-            fn = ctypes.c_void_p()
-            native.check(self.lib.mlc_function(self._mod, symbol.encode(), ctypes.byref(fn)),
-                         f"mlc_function({symbol})")
-            self.functions[symbol] = fn.value
+        for (_, path), table in zip(objects, (self.launch_table, self.product_table)):
+            self._load(path.read_bytes(), sorted({s.symbol for s in table.values()}))
         self._plans: list[ctypes.c_void_p] = []
         self._arena_tensor: torch.Tensor | None = None
         self._static_arena = bool(getattr(cfg, "static_arena", False))
@@ -105,6 +104,18 @@ class HipRuntime:
             word = ctypes.c_void_p()
             native.check(self.lib.mlc_error_word(self._ctx, ctypes.byref(word)), "mlc_error_word")
             self._error_word = word.value
+
+    def _load(self, image: bytes, symbols: list[str]) -> None:
+        mod = ctypes.c_void_p()
+        buf = ctypes.create_string_buffer(image, len(image))
+        native.check(self.lib.mlc_module_load(self._ctx, buf, len(image), ctypes.byref(mod)),
+                     "mlc_module_load")
+        self._mods.append(mod)
+        for symbol in symbols:
+            fn = ctypes.c_void_p()
+            native.check(self.lib.mlc_function(mod, symbol.encode(), ctypes.byref(fn)),
+                         f"mlc_function({symbol})")
+            self.functions[symbol] = fn.value
 
     # -- the reference seam ---------------------------------------------------
 
@@ -135,7 +146,15 @@ class HipRuntime:
     def bind_native_extern(self, k: ExternKernel, buffers: dict[str, torch.Tensor]) -> Bound | None:
         """An extern op this module implements natively (``aten.embedding``),
         resolved like a generated kernel; ``None`` leaves it to the library."""
-        spec = self.launch_table.get(k.name)
+        return self._bind_extern(k, self.launch_table.get(k.name), buffers)
+
+    def bind_product(self, k: ExternKernel, buffers: dict[str, torch.Tensor]) -> Bound | None:
+        """A matrix product this module runs in the library's place, resolved
+        like a generated kernel; ``None`` leaves it to the library."""
+        return self._bind_extern(k, self.product_table.get(k.name), buffers)
+
+    def _bind_extern(self, k: ExternKernel, spec: LaunchSpec | None,
+                     buffers: dict[str, torch.Tensor]) -> Bound | None:
         if spec is None:
             return None
         ptrs = []
@@ -318,9 +337,9 @@ class HipRuntime:
         if getattr(self, "_ctx", None) is not None and self._ctx.value:
             lib.mlc_ctx_destroy(self._ctx)
             self._ctx = None
-        if getattr(self, "_mod", None) is not None and self._mod.value:
-            lib.mlc_module_unload(self._mod)
-            self._mod = None
+        for mod in getattr(self, "_mods", []):
+            lib.mlc_module_unload(mod)
+        self._mods = []
 
     def __del__(self) -> None:
         try:

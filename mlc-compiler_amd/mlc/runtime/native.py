@@ -16,6 +16,7 @@ raises, so nothing can silently run elsewhere.
 
 from __future__ import annotations
 
+import concurrent.futures
 import ctypes
 import functools
 import hashlib
@@ -23,6 +24,7 @@ import os
 import pathlib
 import shutil
 import subprocess
+import threading
 
 PKG = pathlib.Path(__file__).resolve().parents[1]          # .../mlc
 ROOT = PKG.parent                                           # .../mlc-compiler_amd
@@ -183,12 +185,18 @@ def compile_code_object(source: str) -> tuple[pathlib.Path, pathlib.Path]:
     src = d / f"mlc_kernels_{key}.hip"
     obj = d / f"mlc_kernels_{key}.hsaco"
     if not src.exists() or src.read_text() != source:
-        tmp = src.with_name(src.name + f".{os.getpid()}.tmp")
+        tmp = src.with_name(src.name + f".{os.getpid()}.{threading.get_ident()}.tmp")
         tmp.write_text(source)
         tmp.replace(src)
     if not obj.exists():
-        tmp = obj.with_name(obj.name + f".{os.getpid()}.tmp")
+        tmp = obj.with_name(obj.name + f".{os.getpid()}.{threading.get_ident()}.tmp")
         _run([hipcc(), "--genco", *HIP_FLAGS, f"-I{TEMPLATES}", "-x", "hip", str(src),
               "-o", str(tmp)])
         tmp.replace(obj)
     return src, obj
+
+
+def compile_code_objects(sources: list[str]) -> list[tuple[pathlib.Path, pathlib.Path]]:
+    """``compile_code_object`` of each source, the compiler runs side by side."""
+    with concurrent.futures.ThreadPoolExecutor(max(1, len(sources))) as pool:
+        return list(pool.map(compile_code_object, sources))

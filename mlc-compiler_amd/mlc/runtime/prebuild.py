@@ -19,7 +19,7 @@ import torch
 
 from ..api import build_pipeline
 from ..bench.workloads import WORKLOADS, make
-from ..codegen.hip_backend import build_module
+from ..codegen.hip_backend import build_module, build_products
 from ..config import Config
 from ..ir.capture import capture
 from . import native
@@ -55,7 +55,9 @@ def prebuild(items=None, verbose: bool = True) -> None:
         graph = capture(model, args)
         schedule = build_pipeline(graph, cfg)
         module = build_module(schedule, cfg)
-        _, obj = native.compile_code_object(module.source)
+        products = build_products(schedule)
+        (_, obj), *_ = native.compile_code_objects(
+            [module.source] + ([products.source] if products.launches else []))
         if verbose:
             print(f"prebuild {key} max_row={cfg.max_persistent_row}: {len(module.functions)} "
                   f"functions -> {obj.name} ({time.time() - t0:.1f}s)", flush=True)

@@ -1,0 +1,155 @@
+"""Native matrix products in the place of library GEMMs: which calls take
+which form, and both forms at the edges of their tiles, strides and types."""
+
+import pytest
+import torch
+
+import mlc
+from mlc.api import build_pipeline
+from mlc.codegen.hip_gemm import choose_tile, plan_product
+from mlc.config import Config
+from mlc.ir.capture import capture
+from mlc.kernels import ExternKernel
+from mlc.runtime.executor import ProductCall
+
+CFG = Config(cuda_graphs=False, gemm_epilogue=True)
+HALF_ULP = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 0.0}
+
+
+class Linear(torch.nn.Module):
+    def forward(self, x, w):
+        return torch.mm(x, w.t())
+
+
+class Biased(torch.nn.Module):
+    def forward(self, x, w, bias):
+        return torch.mm(x, w.t()) + bias
+
+
+class Batched(torch.nn.Module):
+    def __init__(self, a_order, b_order):
+        super().__init__()
+        self.a_order, self.b_order = a_order, b_order
+
+    def forward(self, a, b):
+        return torch.bmm(a.permute(self.a_order), b.permute(self.b_order))
+
+
+def _plans(model, args):
+    sched = build_pipeline(capture(model, args), CFG)
+    return [plan_product(k) for k in sched.kernels if isinstance(k, ExternKernel)]
+
+
+def _form(model, *args):
+    plan, = _plans(model, args)
+    return None if plan is None else plan.form[0]
+
+
+def test_which_calls_run_natively():
+    def half(*s):
+        return torch.zeros(*s, dtype=torch.float16)
+
+    assert _form(Linear(), half(128, 768), half(768, 768)) == "tiled"
+    assert _form(Linear(), half(1, 64), half(48, 64)) == "tiled"
+    assert _form(Linear(), half(16384, 768), half(3072, 768)) is None      # past the flops line
+    assert _form(Linear(), half(128, 768), half(50257, 768)) is None       # a vocabulary head
+    assert _form(Linear(), half(128, 100), half(96, 100)) is None          # k not in whole pieces
+    assert _form(Linear(), torch.zeros(64, 64, dtype=torch.float64),
+                 torch.zeros(64, 64, dtype=torch.float64)) is None
+    heads = half(12, 128, 64)
+    assert _form(Batched((0, 1, 2), (0, 2, 1)), heads, heads) == "tiled"
+    assert _form(Batched((0, 1, 2), (0, 1, 2)), half(12, 128, 128), heads) == "staged"
+    assert _form(Batched((0, 1, 2), (0, 1, 2)), half(6, 197, 197), half(6, 197, 64)) == "staged"
+    assert _form(Batched((0, 1, 2), (0, 1, 2)), half(64, 1024, 1024), half(64, 1024, 64)) is None
+
+
+@pytest.mark.parametrize("size", [2, 4])
+def test_every_tile_splits_its_product(size):
+    """The tile chosen for any size divides among its waves and its k-splits
+    and fits LDS (the template's own static conditions)."""
+    for M in (1, 2, 15, 16, 17, 33, 64, 100, 128, 197, 300, 512, 1182, 2048):
+        for N in (1, 16, 48, 64, 197, 768, 2304, 3072):
+            for K in (128 // size * n for n in (1, 2, 3, 5, 7, 8, 12, 48)):
+                for batches in (1, 12):
+                    tile, pieces = choose_tile(M, N, K, batches, size), K * size // 128
+                    if tile is None:  # few fp32 rows need a k-split of 4
+                        assert size == 4 and M <= 128 and pieces % 4
+                        continue
+                    TM, TN, WM, WN, WK, stages = tile
+                    assert pieces % WK == 0 and (TM + TN) % (8 * WM * WN) == 0
+                    assert TM % (16 * WM) == 0 and TN % (16 * WN) == 0 and WM * WN * WK <= 16
+                    ring = min(stages, pieces // WK) * WK * (TM + TN) * 128
+                    assert 2 <= stages <= 4 and ring <= 160 * 1024
+                    assert WK == 1 or WK * TM * (TN + 4) * 4 <= 160 * 1024
+
+
+def _check(model, args, want, magnitude, K):
+    """Within half an ulp of the storage type plus the bound of an fp32 sum of
+    K terms in any order, K 2^-24 sum |a b|."""
+    compiled = mlc.compile(model, args, CFG)
+    got = compiled(*args)
+    torch.cuda.synchronize()
+    calls = [p for kind, p in compiled._plan if kind == "extern"]
+    assert calls and all(isinstance(c, ProductCall) for c in calls)
+    got = got.double().cpu()
+    assert torch.isfinite(got).all()
+    bound = HALF_ULP[args[0].dtype] * want.abs() + (K + 2) * 2.0 ** -24 * magnitude + 2.0 ** -25
+    assert ((got - want).abs() <= bound).all(), ((got - want).abs() / bound).max()
+
+
+def _inside(rows, cols, pad, dtype):
+    """A [rows, cols] view with NaN all around it: nothing outside may count."""
+    whole = torch.full((rows + 2, cols + 2 * pad), float("nan"))
+    whole[1:-1, pad:pad + cols] = torch.randn(rows, cols)
+    return whole.to(dtype).cuda()[1:-1, pad:pad + cols]
+
+
+DTYPES = [torch.float16, torch.bfloat16, torch.float32]
+
+
+class Inner(torch.nn.Module):
+    """The same over views cut out of wider buffers inside the program."""
+
+    def forward(self, x, w):
+        return torch.mm(x[1:-1, 8:-8], w[1:-1, 8:-8].t())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", [(1, 16, 64), (17, 50, 320), (128, 768, 3072), (130, 2304, 768),
+                                   (525, 512, 512), (600, 770, 192)])
+def test_tiled(shape, dtype):
+    M, N, K = shape
+    torch.manual_seed(0)
+    x, w = _inside(M, K, 8, dtype)._base, _inside(N, K, 8, dtype)._base
+    a, b = x[1:-1, 8:-8].double().cpu(), w[1:-1, 8:-8].double().cpu()
+    _check(Inner(), (x, w), a @ b.t(), a.abs() @ b.abs().t(), K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_bias_is_added_before_the_rounding(dtype):
+    torch.manual_seed(0)
+    x, w, bias = (torch.randn(*s).to(dtype).cuda() for s in ((70, 256), (100, 256), (100,)))
+    a, b = x.double().cpu(), w.double().cpu()
+    want = a @ b.t() + bias.double().cpu()
+    _check(Biased(), (x, w, bias), want, a.abs() @ b.abs().t() + want.abs(), 256)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("orders", [((0, 1, 2), (0, 1, 2)), ((0, 1, 2), (0, 2, 1)),
+                                    ((0, 2, 1), (0, 1, 2)), ((1, 0, 2), (1, 2, 0)),
+                                    ((2, 0, 1), (1, 0, 2))])
+@pytest.mark.parametrize("shape", [(5, 17, 64, 33), (2, 65, 197, 128), (1, 1, 1, 1)])
+def test_batched_in_every_order(shape, orders, dtype):
+    B, M, N, K = shape
+    torch.manual_seed(0)
+    args = []
+    for order, full in zip(orders, ((B, M, K), (B, K, N))):
+        stored = [0, 0, 0]
+        for at, axis in enumerate(order):
+            stored[axis] = full[at]
+        args.append(torch.randn(*stored).to(dtype).cuda())
+    a, b = (t.double().cpu().permute(o) for t, o in zip(args, orders))
+    _check(Batched(*orders), tuple(args), a @ b, a.abs() @ b.abs(), K)
