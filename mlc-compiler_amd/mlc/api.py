@@ -21,6 +21,7 @@ from .passes.fusion import plan
 from .passes.horizontal import merge_parallel_gemms
 from .passes.layout import fold_relayout_copies
 from .passes.memory_planning import plan_memory
+from .passes.products import merge_products
 
 
 def compile(model: torch.nn.Module, example_inputs: Sequence[torch.Tensor],
@@ -52,6 +53,8 @@ def build_pipeline(graph, cfg: Config) -> Schedule:
         fold_bias_epilogues(schedule)
     if cfg.fused_attention:
         fuse_attention(schedule)
+    if cfg.gemm_epilogue:
+        merge_products(schedule)
     plan_memory(graph, schedule, cfg)
     return schedule
 

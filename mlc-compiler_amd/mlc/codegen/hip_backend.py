@@ -1812,11 +1812,17 @@ def build_module(schedule: Schedule, cfg: Config) -> Module:
     return _module(((k.name, emit_kernel(k, cfg)) for k in schedule.kernels), PRELUDE)
 
 
-def build_products(schedule: Schedule) -> Module:
+def build_products(schedule: Schedule) -> tuple[Module, dict[str, LaunchSpec]]:
     """The same for the library calls that run as native matrix products
     (``hip_gemm``), a module of their own: its text depends on the products'
-    sizes alone, so schedules of one model share its code object."""
-    from .hip_gemm import emit_product
+    sizes alone, so schedules of one model share its code object. The second
+    table holds the groups that run as one launch (``Schedule.merged``), by
+    their first kernel's name."""
+    from .hip_gemm import emit_group, emit_product
 
-    return _module(((k.name, emit_product(k)) for k in schedule.kernels
-                    if isinstance(k, ExternKernel)), PRELUDE + '#include "mlc_gemm.h"\n')
+    merged = {schedule.kernels[i].name: emit_group(schedule.kernels[i], parts)
+              for i, (_, parts) in schedule.merged.items()}
+    alone = [(k.name, emit_product(k)) for k in schedule.kernels
+             if isinstance(k, ExternKernel) and k.name not in merged]
+    module = _module([*alone, *merged.items()], PRELUDE + '#include "mlc_gemm.h"\n')
+    return module, {name: module.launches.pop(name) for name in merged}

@@ -30,8 +30,10 @@ from dataclasses import dataclass
 import torch
 
 from ..ir.graph import Value
+from ..ir.scalar import Call
 from ..kernels import ExternKernel
-from .hip_backend import STORAGE, LaunchSpec, itemsize
+from .hip_backend import (STORAGE, LaunchSpec, Renderer, _subexprs as subexprs, fp16_rounded,
+                          half_inputs, itemsize, value_types_of)
 
 CUS, XCDS = 256, 8
 LDS_BYTES = 160 * 1024
@@ -44,8 +46,18 @@ TILES = ((16, 16, 1, 1, (1, 2, 4)), (16, 32, 1, 2, (2, 4)), (16, 32, 1, 1, (3,))
          (96, 96, 2, 2, (1,)), (128, 96, 2, 2, (1,)), (128, 128, 2, 4, (1,)),
          (128, 192, 2, 4, (1,)))
 #: floating-point operations up to which the tiled form is at least the
-#: library's speed (the table above), by element size
+#: library's speed (the table above), by element size; and for a square-ish
+#: weight, where it holds on (16384x768x768 fp16: 25.0 us, tiled 23.5)
 TILED_FLOPS = {2: 10e9, 4: 2.2e9}
+NARROW, NARROW_FLOPS = 1024, {2: 20e9, 4: 2.2e9}
+#: the same with pointwise kernels in the epilogue, against the library and
+#: those kernels after it (fp16): 8192x3072x768 + bias + GELU 58 us against
+#: 46 + 19, 16384x3072x768 111 against 74 + 36; the bias and re-layout of
+#: 16384x2304x768 cost 3 us on 68 against 67 + 29; 16384x768x3072 + bias +
+#: residual 85 against 69 + 12. An epilogue with a transcendental is arithmetic
+#: that nothing overlaps once a CU holds one large tile.
+MERGED_FLOPS, MERGED_MATH_FLOPS = 60e9, 40e9
+TRANSCENDENTAL = {"erf", "exp", "tanh", "sigmoid", "sin", "cos", "log", "pow"}
 #: widest product measured: a vocabulary head streams its weights, where the
 #: library's larger tiles win
 MAX_COLUMNS = 4096
@@ -111,7 +123,8 @@ def tile_cost(M: int, N: int, K: int, batches: int, size: int, tile: tuple) -> f
 
 
 def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None:
-    """The cheapest tile by ``tile_cost``, with the deepest ring that fits LDS.
+    """The cheapest tile by ``tile_cost``, with the deepest ring that fits LDS
+    (half of it where a CU has more than one tile to do).
 
     In fp32 a k-split of 4 is kept up to 128 rows, where the library sums k in
     as many parts: fewer, longer sums would be further from float64 than it
@@ -128,8 +141,16 @@ def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None
             if pieces % WK or WK < min(fewest, pieces):
                 continue
             steps = pieces // WK
-            stages = next((n for n in (4, 3, 2)
-                           if min(n, steps) * WK * (TM + TN) * 128 <= LDS_BYTES), None)
+
+            def deepest(lds: int):
+                return next((n for n in (4, 3, 2)
+                             if min(n, steps) * WK * (TM + TN) * 128 <= lds), None)
+
+            # several tiles per CU: two workgroups at a time, one's epilogue
+            # and first loads under the other's products
+            tiles = batches * -(-M // TM) * -(-N // TN)
+            crowded = -(-tiles // XCDS) > CUS // XCDS
+            stages = (deepest(LDS_BYTES // 2) if crowded else None) or deepest(LDS_BYTES)
             if stages is None:
                 continue
             tile = (TM, TN, WM, WN, WK, min(stages, max(2, steps)))
@@ -144,9 +165,10 @@ def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None
 STAGED_FLOPS = 2e9
 
 
-def plan_product(k: ExternKernel) -> Product | None:
+def plan_product(k: ExternKernel, merged_flops: float = 0.0) -> Product | None:
     """How a library call's product runs natively, or ``None`` to leave it to
-    the library."""
+    the library. ``merged_flops``: the line where pointwise kernels run in its
+    epilogue, which pays for itself where the product alone does not."""
     node = k.node
     op = node.op
     if op not in ("aten.mm.default", "aten.addmm.default", "aten.bmm.default") or node.kwargs:
@@ -179,7 +201,10 @@ def plan_product(k: ExternKernel) -> Product | None:
     size = itemsize(x.dtype)
     flops = 2.0 * batches * M * N * K
     E = 16 // size
-    if (K * size % 128 == 0 and N <= MAX_COLUMNS and flops <= TILED_FLOPS[size]
+    line = (NARROW_FLOPS if max(N, K) <= NARROW else TILED_FLOPS)[size]
+    if size == 2:
+        line = max(line, merged_flops)
+    if (K * size % 128 == 0 and N <= MAX_COLUMNS and flops <= line
             and a.aligned(E, batches) and b.aligned(E, batches)):
         tile = choose_tile(M, N, K, batches, size)
         if tile is not None:
@@ -199,29 +224,78 @@ def staged_tile(M: int, N: int, batches: int) -> tuple[int, int]:
     return TM, TN
 
 
+@dataclass(frozen=True)
+class _Source:
+    """The pieces of a product's kernel around its epilogue."""
+
+    p: Product
+
+    @property
+    def storage(self) -> str:
+        return STORAGE[self.p.a.value.dtype]
+
+    @property
+    def tile(self) -> tuple[int, int]:
+        return self.p.form[1], self.p.form[2]
+
+    @property
+    def threads(self) -> int:
+        return 64 * math.prod(self.p.form[3:6]) if self.p.form[0] == "tiled" else 256
+
+    @property
+    def grid(self) -> int:
+        return XCDS * -(-self.p.batches * self._tiles[0] * self._tiles[1] // XCDS)
+
+    @property
+    def _tiles(self) -> tuple[int, int]:
+        return -(-self.p.M // self.tile[0]), -(-self.p.N // self.tile[1])
+
+    def head(self, params: list[str]) -> list[str]:
+        p, T = self.p, self.storage
+        params = [f"const {T}* __restrict__ a", f"const {T}* __restrict__ b", *params]
+        L = [f"extern \"C\" __global__ void __launch_bounds__({self.threads}) "
+             f"KERNEL({', '.join(params)}) {{",
+             f"  // {p.form[0]}: {p.batches} x [{p.M} x {p.K}] x [{p.K} x {p.N}], "
+             f"{self.tile[0]} x {self.tile[1]} tiles",
+             "  int z, mt, nt;",
+             f"  if (!mlc::tile_index<{p.batches}, {self._tiles[0]}, {self._tiles[1]}>(z, mt, nt)) return;"]
+        return L + [self.move("a", p.a), self.move("b", p.b)]
+
+    def move(self, name: str, o: Operand) -> str:
+        """``name`` at this batch's first element."""
+        return f"  {name} += (int64_t)z * {o.batch if self.p.batches > 1 else 0} + {o.base};"
+
+    def tail(self) -> list[str]:
+        p, T = self.p, self.storage
+        (TM, TN), E = self.tile, 16 // itemsize(p.a.value.dtype)
+        if p.form[0] == "tiled":
+            return [f"  mlc::gemm_tile<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.b.row}, "
+                    f"{', '.join(map(str, p.form[1:]))}>(a, b, mt * {TM}, nt * {TN}, store);", "}"]
+        flags = ", ".join(str(o.aligned(E, p.batches) and p.K % E == 0).lower() for o in (p.a, p.b))
+        return [f"  mlc::gemm_staged<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.a.k}, {p.b.row}, {p.b.k}, "
+                f"{TM}, {TN}, {8 * E}, {flags}>(a, b, mt * {TM}, nt * {TN}, store);", "}"]
+
+    def spec(self, kind: str, values: list[Value]) -> LaunchSpec:
+        return LaunchSpec("", self.grid, self.threads, 0,
+                          {"kind": kind, "form": self.p.form,
+                           "buffers": [v.buffer.name for v in values],
+                           "dtypes": [v.buffer.dtype for v in values],
+                           "numels": [v.buffer.numel for v in values]})
+
+
 def emit_product(k: ExternKernel) -> tuple[str, LaunchSpec] | None:
     """Source (with the placeholder name ``KERNEL``) and launch spec of a
     library call's native product, or ``None``."""
     p = plan_product(k)
     if p is None:
         return None
-    T = STORAGE[p.a.value.dtype]
-    E = 16 // itemsize(p.a.value.dtype)
-    form, TM, TN = p.form[:3]
-    mt, nt = -(-p.M // TM), -(-p.N // TN)
-    tiles = p.batches * mt * nt
-    threads = 64 * math.prod(p.form[3:6]) if form == "tiled" else 256
+    src = _Source(p)
+    T = src.storage
     packed = p.N % 4 == 0 and p.out.aligned(4, p.batches)
-    bias = f", const {T}* __restrict__ bias" if p.bias is not None else ""
-    L = [f"extern \"C\" __global__ void __launch_bounds__({threads}) "
-         f"KERNEL(const {T}* __restrict__ a, const {T}* __restrict__ b{bias}, {T}* __restrict__ c) {{",
-         f"  // {form}: {p.batches} x [{p.M} x {p.K}] x [{p.K} x {p.N}], {TM} x {TN} tiles",
-         "  int t;",
-         f"  if (!mlc::tile_index<{tiles}>(t)) return;",
-         f"  const int z = t / {mt * nt}, mt = t % {mt}, nt = t / {mt} % {nt};"]
-    for name, o in (("a", p.a), ("b", p.b), ("c", p.out)):
-        L.append(f"  {name} += (int64_t)z * {o.batch if p.batches > 1 else 0} + {o.base};")
-    L += ["  auto store = [&](int m, int n, mlc::float4v s) {",
+    params = [f"const {T}* __restrict__ bias"] if p.bias is not None else []
+    L = src.head(params + [f"{T}* __restrict__ c"])
+    L += [src.move("c", p.out),
+          "  auto store = [&](int m, int n, mlc::float4v s) {",
           "    float v[4] = {s[0], s[1], s[2], s[3]};"]
     if p.bias is not None:
         L += ["#pragma unroll",
@@ -229,17 +303,106 @@ def emit_product(k: ExternKernel) -> tuple[str, LaunchSpec] | None:
               f"v[i] += mlc::ld(bias + {p.bias.layout.offset} + n + i);"]
     L += [f"    mlc::store4<{T}, {p.M}, {p.N}, {p.out.row}, {str(packed).lower()}>(c, m, n, v);",
           "  };"]
-    if form == "tiled":
-        L.append(f"  mlc::gemm_tile<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.b.row}, "
-                 f"{', '.join(map(str, p.form[1:]))}>(a, b, mt * {TM}, nt * {TN}, store);")
-    else:
-        flags = ", ".join(str(o.aligned(E, p.batches) and p.K % E == 0).lower() for o in (p.a, p.b))
-        L.append(f"  mlc::gemm_staged<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.a.k}, {p.b.row}, {p.b.k}, "
-                 f"{TM}, {TN}, {8 * E}, {flags}>(a, b, mt * {TM}, nt * {TN}, store);")
-    L.append("}")
     values = [p.a.value, p.b.value, *([p.bias] if p.bias is not None else []), p.out.value]
-    spec = LaunchSpec("", XCDS * -(-tiles // XCDS), threads, 0,
-                      {"kind": "gemm", "form": p.form, "buffers": [v.buffer.name for v in values],
-                       "dtypes": [v.buffer.dtype for v in values],
-                       "numels": [v.buffer.numel for v in values]})
-    return "\n".join(L), spec
+    return "\n".join(L + src.tail()), src.spec("gemm", values)
+
+
+# --------------------------------------------------------------------------
+# products with the pointwise kernels after them
+# --------------------------------------------------------------------------
+
+def plan_group(k: ExternKernel, parts) -> Product | None:
+    """The product of a group that runs as one launch (``passes/products``),
+    or ``None`` where the kernels stay apart."""
+    if any(a.buffer.numel >= 2 ** 31 for part in parts
+           for a in (*part.kernel.inputs, *part.kernel.outputs)):
+        return None
+    calls = {e.fn for part in parts for _, x in part.kernel.body for e in subexprs(x)
+             if isinstance(e, Call)}
+    return plan_product(k, MERGED_MATH_FLOPS if calls & TRANSCENDENTAL else MERGED_FLOPS)
+
+
+def _place(terms, var: str) -> str:
+    """Index of an output element from one coordinate (``Part.m_terms``),
+    in unsigned arithmetic: most sizes are powers of two, so their divisions
+    are shifts."""
+    top = max((size * step for size, step, _ in terms), default=1)
+    parts = []
+    for size, step, stride in terms:
+        t = var if step == 1 else f"{var} / {step}u"
+        t = t if size * step == top else f"{t} % {size}u"
+        parts.append(f"({t}) * {stride}u")
+    return " + ".join(parts) or "0u"
+
+
+def _part_lines(part, i: int, N: int, TN: int) -> list[str]:
+    """One pointwise kernel's work on four consecutive columns ``n`` of row
+    ``m``: ``x`` holds the product, already rounded to its storage type.
+    Where its columns are whole tiles, which kernel applies is one scalar
+    branch per workgroup."""
+    k = part.kernel
+    out = k.outputs[0]
+    if part.lo == 0 and part.hi == N:
+        test = "true"
+    elif part.lo % TN == 0 and part.hi % TN == 0:
+        test = f"nt >= {part.lo // TN} && nt < {part.hi // TN}"
+    else:
+        test = f"n >= {part.lo} && n < {part.hi}"
+    L = [f"    if ({test}) {{", f"      const uint32_t q = n - {part.lo}, row = m;"]
+    names: list[str] = []
+    for slot, (a, read) in enumerate(zip(k.inputs, part.reads)):
+        if read is None:
+            names.append("x[j]")
+            continue
+        at = f"p{i}_{slot} + (row * {read.row}u + {read.base}u" + (" + q)" if read.col else ")")
+        if read.col:
+            packed = read.row % 4 == 0 and read.base % 4 == 0
+            L.append(f"      float v{slot}[4];" + (f" mlc::load_pack<4>(v{slot}, {at});" if packed else
+                     f" for (int j = 0; j < 4; ++j) v{slot}[j] = mlc::ld({at} + j);"))
+            names.append(f"v{slot}[j]")
+        else:
+            L.append(f"      const float v{slot} = mlc::ld({at});")
+            names.append(f"v{slot}")
+    types: dict[str, str] = {}
+    r = Renderer(lambda s: (names[s], "float"), lambda n: (n, types[n]), half_inputs(k), dict(k.body),
+                 fp16_rounded(k), value_types_of(k))
+    L += ["      float o[4];", "#pragma unroll", "      for (int j = 0; j < 4; ++j) {"]
+    for name, expr in k.body:
+        code, types[name] = r.bind(name, expr)
+        L.append(f"        const {types[name]} {name} = {code};")
+    code, _ = r.store(k.out_expr[out.value.name], out.dtype == torch.float16)
+    inner = next((t for t in part.n_terms if t[1] == 1), (1, 1, 1))
+    terms = (*part.m_terms, *part.n_terms)
+    packed = inner[2] == 1 and all(t is inner or t[2] % 4 == 0 for t in terms) and inner[0] % 4 == 0
+    L += [f"        o[j] = {code};", "      }",
+          f"      {STORAGE[out.dtype]}* w = o{i} + (({_place(part.m_terms, 'row')}) "
+          f"+ ({_place(part.n_terms, 'q')}));"]
+    if packed:
+        L.append("      mlc::store_pack<4>(w, o);")
+    else:
+        L += ["#pragma unroll",
+              f"      for (int j = 0; j < 4; ++j) mlc::st(w + j * {inner[2]}, o[j]);"]
+    return L + ["    }"]
+
+
+def emit_group(k: ExternKernel, parts) -> tuple[str, LaunchSpec]:
+    """A product and the pointwise kernels after it as one kernel."""
+    p = plan_group(k, parts)
+    src = _Source(p)
+    T = src.storage
+    params, values = [], [p.a.value, p.b.value]
+    for i, part in enumerate(parts):
+        for slot, (a, read) in enumerate(zip(part.kernel.inputs, part.reads)):
+            if read is not None:
+                params.append(f"const {STORAGE[a.dtype]}* __restrict__ p{i}_{slot}")
+                values.append(a.value)
+        out = part.kernel.outputs[0]
+        params.append(f"{STORAGE[out.dtype]}* __restrict__ o{i}")
+        values.append(out.value)
+    L = src.head(params) + ["  auto store = [&](int m, int n, mlc::float4v s) {"]
+    if p.M % src.tile[0] or p.N % src.tile[1]:
+        L.append(f"    if (m >= {p.M} || n >= {p.N}) return;")
+    L.append("    const float x[4] = {" + ", ".join(f"mlc::ld_of<{T}>(s[{j}])" for j in range(4)) + "};")
+    for i, part in enumerate(parts):
+        L += _part_lines(part, i, p.N, src.tile[1])
+    return "\n".join(L + ["  };"] + src.tail()), src.spec("gemm+pointwise", values)

@@ -11,14 +11,23 @@
 
 namespace mlc {
 
-// This workgroup's tile of a TILES-tile product, false past the last one.
-// Workgroups go to the 8 XCDs in turn, so each XCD takes a contiguous eighth
-// of the tiles: with the row tile running fastest, the tiles that share B's
-// rows (the weights) share an L2.
-template <int TILES> __device__ __forceinline__ bool tile_index(int& t) {
-  constexpr int PER = (TILES + 7) / 8;
-  t = (int)(blockIdx.x % 8) * PER + (int)(blockIdx.x / 8);
-  return (int)(blockIdx.x / 8) < PER && t < TILES;
+// This workgroup's (row, column) tile of BATCHES products of MT x NT tiles,
+// false past the last one. Workgroups go to the 8 XCDs in turn, so each XCD
+// takes a contiguous eighth of the tiles: bands of up to 8 row tiles, columns
+// outside rows, so that the tiles of one XCD at a time share few rows of A and
+// few of B and find them in its L2. (With whole columns instead, 64 row tiles
+// read A from memory once per column: 16384x768x3072 fp16 took 111 us, 73 now.)
+template <int BATCHES, int MT, int NT>
+__device__ __forceinline__ bool tile_index(int& z, int& mt, int& nt) {
+  constexpr int TILES = BATCHES * MT * NT, PER = (TILES + 7) / 8, BAND = MT < 8 ? MT : 8;
+  const int i = (int)(blockIdx.x / 8), t = (int)(blockIdx.x % 8) * PER + i;
+  if (i >= PER || t >= TILES) return false;
+  z = t / (MT * NT);
+  const int u = t % (MT * NT), band = u / (BAND * NT), v = u % (BAND * NT);
+  const int rows = MT - band * BAND < BAND ? MT - band * BAND : BAND;
+  mt = band * BAND + v % rows;
+  nt = v / rows;
+  return true;
 }
 
 template <class T> struct mma_type;
@@ -70,15 +79,16 @@ template <class T, int M, int N, int K, int LDA, int LDB, int TM, int TN, int WM
 __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __restrict__ b,
                                           int m0, int n0, Epi epi) {
   typedef typename mma_type<T>::frag frag;
-  constexpr int BK = 128 / sizeof(T), E = 16 / sizeof(T);
+  constexpr int PIECE = 128, BK = PIECE / sizeof(T);     // bytes and elements of k per stage
+  constexpr int SLOTS = PIECE / 16, RPL = 64 / SLOTS;  // rows per load instruction
   constexpr int GW = WM * WN;                          // waves per k-group
   constexpr int IT = K / (BK * WK);                    // stages per k-group
-  constexpr int ROWS = TM + TN, LPW = ROWS / 8 / GW;   // 8 rows per load instruction
+  constexpr int ROWS = TM + TN, LPW = ROWS / RPL / GW;
   constexpr int RA = TM / WM / 16, RB = TN / WN / 16;
-  static_assert(K % (BK * WK) == 0 && ROWS % (8 * GW) == 0, "tile split");
+  static_assert(K % (BK * WK) == 0 && ROWS % (RPL * GW) == 0, "tile split");
   static_assert(TM % (16 * WM) == 0 && TN % (16 * WN) == 0, "wave split");
   constexpr int RING = IT < NST ? IT : NST;
-  constexpr int STAGE = ROWS * 128;
+  constexpr int STAGE = ROWS * PIECE;
   constexpr int PART = WK > 1 ? WK * TM * (TN + 4) * 4 : 0;
   constexpr int LDS = WK * RING * STAGE > PART ? WK * RING * STAGE : PART;
   __shared__ __attribute__((aligned(1024))) char lds[LDS];
@@ -93,8 +103,8 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
   const char* src[LPW];
 #pragma unroll
   for (int i = 0; i < LPW; ++i) {
-    const int q = w + i * GW, row = q * 8 + (lane >> 3);
-    const int chunk = (lane & 7) ^ ((row >> 1) & 7);
+    const int q = w + i * GW, row = q * RPL + lane / SLOTS;
+    const int chunk = (lane % SLOTS) ^ (row / (16 / SLOTS) % SLOTS);
     const T* p;
     if (row < TM) {
       const int m = m0 + row;
@@ -103,12 +113,12 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
       const int n = n0 + row - TM;
       p = b + (int64_t)(n < N ? n : N - 1) * LDB;
     }
-    src[i] = reinterpret_cast<const char*>(p) + group * (IT * 128) + chunk * 16;
+    src[i] = reinterpret_cast<const char*>(p) + group * (IT * PIECE) + chunk * 16;
   }
   auto load = [&](int it) {
     char* dst = ring + (it % RING) * STAGE + w * 1024;
 #pragma unroll
-    for (int i = 0; i < LPW; ++i) load_to_lds(src[i] + it * 128, dst + i * GW * 1024);
+    for (int i = 0; i < LPW; ++i) load_to_lds(src[i] + it * PIECE, dst + i * GW * 1024);
   };
 
   float4v acc[RA][RB];
@@ -117,23 +127,28 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
 #pragma unroll
     for (int j = 0; j < RB; ++j) acc[i][j] = float4v{0.0f, 0.0f, 0.0f, 0.0f};
 
-  const int swz = r >> 1;
+  const int swz = r / (16 / SLOTS) % SLOTS;
   auto compute = [&](int it) {
     const char* st = ring + (it % RING) * STAGE;
-    const char* sa = st + (wm * (TM / WM) + r) * 128;
-    const char* sb = st + (TM + wn * (TN / WN) + r) * 128;
-#pragma unroll
-    for (int s = 0; s < 2; ++s) {
+    const char* sa = st + (wm * (TM / WM) + r) * PIECE;
+    const char* sb = st + (TM + wn * (TN / WN) + r) * PIECE;
+    constexpr int STEPS = PIECE / 64;
+    frag fa[STEPS][RA], fb[STEPS][RB];
+    auto read = [&](int s) {
       const int at = ((s * 4 + g) ^ swz) * 16;
-      frag fa[RA], fb[RB];
 #pragma unroll
-      for (int i = 0; i < RA; ++i) fa[i] = *reinterpret_cast<const frag*>(sa + i * 2048 + at);
+      for (int i = 0; i < RA; ++i) fa[s][i] = *reinterpret_cast<const frag*>(sa + i * 16 * PIECE + at);
 #pragma unroll
-      for (int j = 0; j < RB; ++j) fb[j] = *reinterpret_cast<const frag*>(sb + j * 2048 + at);
+      for (int j = 0; j < RB; ++j) fb[s][j] = *reinterpret_cast<const frag*>(sb + j * 16 * PIECE + at);
+    };
+    read(0);
+#pragma unroll
+    for (int s = 0; s < STEPS; ++s) {
+      if (s + 1 < STEPS) read(s + 1);  // in flight during this step's products
 #pragma unroll
       for (int i = 0; i < RA; ++i)
 #pragma unroll
-        for (int j = 0; j < RB; ++j) acc[i][j] = mma16(fb[j], fa[i], acc[i][j]);
+        for (int j = 0; j < RB; ++j) acc[i][j] = mma16(fb[s][j], fa[s][i], acc[i][j]);
     }
   };
   // one group of one wave needs no barrier: its stages are its own
@@ -311,6 +326,11 @@ __device__ __forceinline__ void gemm_staged(const T* __restrict__ a, const T* __
 #pragma unroll
     for (int j = 0; j < RB; ++j) epi(m0 + wm + 16 * i + r, n0 + wn + 16 * j + 4 * g, acc[i][j]);
 }
+
+// A product as its storage type T holds it, in an fp32 register.
+template <class T> __device__ __forceinline__ float ld_of(float x) { return x; }
+template <> __device__ __forceinline__ float ld_of<f16>(float x) { return round_f16(x); }
+template <> __device__ __forceinline__ float ld_of<bf16>(float x) { return round_bf16(x); }
 
 // Four consecutive columns of one row, dropped past M and N; 8- or 16-byte
 // stores when every row starts on that boundary.

@@ -184,6 +184,9 @@ class ExternKernel(Kernel):
 class Schedule:
     graph: object
     kernels: list[Kernel] = field(default_factory=list)
+    #: groups of kernels that run as one launch: first index -> (last index,
+    #: parts), ``passes/products``
+    merged: dict = field(default_factory=dict)
     #: set by the planner
     arena_bytes: int = 0
     plan: object | None = None

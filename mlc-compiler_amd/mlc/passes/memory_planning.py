@@ -97,11 +97,14 @@ def compute_live_ranges(graph: Graph, schedule: Schedule) -> list[LiveRange]:
             first.setdefault(buf.name, i)
         last[buf.name] = max(last.get(buf.name, i), i)
 
+    # kernels that run as one launch touch their buffers from its first to its last
+    span = {j: (i, end) for i, (end, _) in schedule.merged.items() for j in range(i, end + 1)}
     for i, k in enumerate(schedule.kernels):
+        begin, end = span.get(i, (i, i))
         for v in k.writes():
-            touch(v.buffer, i, True)
-        for v in k.reads():
-            touch(v.buffer, i, False)
+            touch(v.buffer, begin, True)
+        for v in (*k.writes(), *k.reads()):
+            touch(v.buffer, end, False)
     for v in graph.outputs:  # results outlive the schedule
         by_name.setdefault(v.buffer.name, v.buffer)
         last[v.buffer.name] = len(schedule.kernels)

@@ -339,8 +339,19 @@ class CompiledModel:
             else:
                 plan.append(("kernel", self._module.bind(k, table)))
         self._plan = plan
+        # what a pass runs: a group of kernels that is one launch takes the
+        # place of its members
+        bind_group = getattr(self._module, "bind_group", None)
+        launches, i = [], 0
+        while i < len(plan):
+            if bind_group is not None and i in self.schedule.merged:
+                launches.append(("kernel", bind_group(self.schedule.kernels[i], table)))
+                i = self.schedule.merged[i][0] + 1
+            else:
+                launches.append(plan[i])
+                i += 1
         group = getattr(self._module, "compile_runs", None)
-        self._runs = group(plan) if group is not None else plan
+        self._runs = group(launches) if group is not None else launches
 
     def run_one(self, k, table: dict[str, torch.Tensor]) -> None:
         if isinstance(k, ExternKernel):

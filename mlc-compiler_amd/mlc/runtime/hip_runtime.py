@@ -82,17 +82,18 @@ class HipRuntime:
         self.launch_table: dict[str, LaunchSpec] = self.module.launches
         #: library products that run natively, by kernel name; their module
         #: is loaded beside the generated one when there are any
-        products = build_products(schedule)
+        products, self.group_table = build_products(schedule)
         self.product_table: dict[str, LaunchSpec] = products.launches
         objects = native.compile_code_objects(
-            [self.source] + ([products.source] if products.launches else []))
+            [self.source] + ([products.source] if products.functions else []))
         self.path, self.code_object_path = objects[0]
 
         self._ctx = ctypes.c_void_p()
         native.check(self.lib.mlc_ctx_create(self.index, ctypes.byref(self._ctx)), "mlc_ctx_create")
         self._mods: list[ctypes.c_void_p] = []
         self.functions: dict[str, int] = {}
-        for (_, path), table in zip(objects, (self.launch_table, self.product_table)):
+        for (_, path), table in zip(objects, (self.launch_table,
+                                              {**self.product_table, **self.group_table})):
             self._load(path.read_bytes(), sorted({s.symbol for s in table.values()}))
         self._plans: list[ctypes.c_void_p] = []
         self._arena_tensor: torch.Tensor | None = None
@@ -152,6 +153,10 @@ class HipRuntime:
         """A matrix product this module runs in the library's place, resolved
         like a generated kernel; ``None`` leaves it to the library."""
         return self._bind_extern(k, self.product_table.get(k.name), buffers)
+
+    def bind_group(self, k: ExternKernel, buffers: dict[str, torch.Tensor]) -> Bound:
+        """The group of kernels starting at ``k`` that runs as one launch."""
+        return self._bind_extern(k, self.group_table[k.name], buffers)
 
     def _bind_extern(self, k: ExternKernel, spec: LaunchSpec | None,
                      buffers: dict[str, torch.Tensor]) -> Bound | None:

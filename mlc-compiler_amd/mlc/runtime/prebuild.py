@@ -55,9 +55,9 @@ def prebuild(items=None, verbose: bool = True) -> None:
         graph = capture(model, args)
         schedule = build_pipeline(graph, cfg)
         module = build_module(schedule, cfg)
-        products = build_products(schedule)
+        products, _ = build_products(schedule)
         (_, obj), *_ = native.compile_code_objects(
-            [module.source] + ([products.source] if products.launches else []))
+            [module.source] + ([products.source] if products.functions else []))
         if verbose:
             print(f"prebuild {key} max_row={cfg.max_persistent_row}: {len(module.functions)} "
                   f"functions -> {obj.name} ({time.time() - t0:.1f}s)", flush=True)

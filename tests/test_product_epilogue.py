@@ -1,0 +1,159 @@
+"""Products that absorb the pointwise kernels after them
+(``Config.gemm_epilogue``): which groups form, that a tile's coordinates give
+every operand the element its own index map names, and the results."""
+
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+import mlc
+from mlc.api import build_pipeline
+from mlc.config import Config
+from mlc.ir.capture import capture
+from mlc.kernels import ExternKernel
+
+ALL = Config(cuda_graphs=False, merge_parallel_gemms=True, gemm_epilogue=True,
+             layout_selection=True, fused_attention=True)
+
+
+class Mlp(nn.Module):
+    def __init__(self, w=64, f=192):
+        super().__init__()
+        self.up, self.down = nn.Linear(w, f), nn.Linear(f, w)
+
+    def forward(self, x):
+        return x + self.down(F.gelu(self.up(x))) * 0.5
+
+
+class Heads(nn.Module):
+    """q, k and v re-laid out per head, V transposed by the attention."""
+
+    def __init__(self, w=128, h=2):
+        super().__init__()
+        self.h, self.qkv = h, nn.Linear(w, 3 * w)
+
+    def forward(self, x):
+        b, n, w = x.shape
+        q, k, v = (t.view(b, n, self.h, w // self.h).transpose(1, 2)
+                   for t in self.qkv(x).chunk(3, -1))
+        return ((q @ k.transpose(-2, -1)) / 8.0).softmax(-1) @ v
+
+
+class RowScale(nn.Module):
+    """An operand that moves with the row alone, and a sliced (pitched) one."""
+
+    def __init__(self):
+        super().__init__()
+        self.w = nn.Parameter(torch.randn(128, 64) * 0.1)
+
+    def forward(self, x, scale, wide):
+        return torch.mm(x, self.w.t()) * scale + wide[:, 4:132]
+
+
+class Transposed(nn.Module):
+    """The product read column by column."""
+
+    def __init__(self):
+        super().__init__()
+        self.w = nn.Parameter(torch.randn(96, 64) * 0.1)
+
+    def forward(self, x):
+        y = torch.mm(x, self.w.t())
+        return (y.t() + 1.0).contiguous()
+
+
+class TwiceRead(nn.Module):
+    """A second reader that is not pointwise: no group."""
+
+    def __init__(self):
+        super().__init__()
+        self.w = nn.Parameter(torch.randn(96, 64) * 0.1)
+
+    def forward(self, x):
+        y = torch.mm(x, self.w.t())
+        return torch.relu(y) * 2.0, y.sum(-1)
+
+
+def cases(dtype=torch.float16):
+    def r(*s):
+        return torch.randn(*s).to(dtype)
+
+    torch.manual_seed(0)
+    return [("mlp", Mlp(), (r(37, 64),), 2), ("mlp b2", Mlp(), (r(2, 16, 64),), 2),
+            ("heads", Heads(), (r(2, 32, 128),), 1), ("row scale", RowScale(), (r(33, 64), r(33, 1), r(33, 140)), 1),
+            ("transposed", Transposed(), (r(40, 64),), None), ("twice", TwiceRead(), (r(40, 64),), 0)]
+
+
+def _schedule(model, args):
+    return build_pipeline(capture(model.to(args[0].dtype), args), ALL)
+
+
+@pytest.mark.parametrize("at", range(6))
+def test_groups_and_their_addresses(at):
+    name, model, args, groups = cases()[at]
+    sched = _schedule(model, args)
+    if groups is not None:
+        assert len(sched.merged) == groups, sched
+    for i, (end, parts) in sched.merged.items():
+        y = sched.kernels[i].outputs[0]
+        M, N = y.shape
+        assert isinstance(sched.kernels[i], ExternKernel) and end == i + len(parts)
+        for part in parts:
+            k = part.kernel
+            own = next(a for a, read in zip(k.inputs, part.reads) if read is None)
+            for idx in range(k.numel):
+                m, n = divmod(own.index.evaluate(idx=idx), N)
+                assert part.lo <= n < part.hi
+                place = sum(m // p % s * t for s, p, t in part.m_terms) + \
+                    sum((n - part.lo) // p % s * t for s, p, t in part.n_terms)
+                assert place == idx, name
+                for a, read in zip(k.inputs, part.reads):
+                    if read is not None:
+                        assert a.index.evaluate(idx=idx) == \
+                            read.base + read.row * m + read.col * (n - part.lo), name
+
+
+def test_a_group_keeps_its_buffers_alive_throughout():
+    """The down projection's residual and input outlive the group's output's
+    first write: no two of them share arena bytes."""
+    sched = _schedule(*cases()[1][1:3])
+    plan = sched.plan
+    for i, (end, parts) in sched.merged.items():
+        names = {v.buffer.name for k in sched.kernels[i:end + 1] for v in (*k.reads(), *k.writes())}
+        spans = sorted((plan.offsets[n], plan.offsets[n] + plan.live_ranges[n].size)
+                       for n in names if n in plan.offsets)
+        assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("at", range(5))
+def test_results(at, dtype):
+    """Against float64 of the same values: a few roundings of the storage type
+    over sums of at most 192 products."""
+    name, model, args, _ = cases(dtype)[at]
+    model = model.to(dtype)
+    want = model.double()(*(a.double() for a in args))
+    model = model.to(dtype).cuda()
+    compiled = mlc.compile(model, tuple(a.cuda() for a in args), ALL)
+    got = compiled(*(a.cuda() for a in args))
+    torch.cuda.synchronize()
+    runs = [kind for kind, _ in compiled._runs]
+    if name not in ("twice", "transposed"):
+        assert len(compiled.schedule.merged) >= 1 and "extern" not in runs
+    ulp = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    err = (got.double().cpu() - want).abs().max() / want.abs().max()
+    assert err <= 4 * ulp, (name, err)
+
+
+@pytest.mark.gpu
+def test_a_replayed_graph_gives_the_uncaptured_result():
+    name, model, args, _ = cases()[2]
+    model, args = model.half().cuda(), tuple(a.cuda() for a in args)
+    want = mlc.compile(model, args, ALL)(*args).clone()
+    compiled = mlc.compile(model, args, ALL.replace(cuda_graphs=True))
+    for _ in range(3):
+        assert torch.equal(compiled(*args), want)
+        torch.cuda.synchronize()
+        torch.zeros(1 << 16, device="cuda").add_(1)
