@@ -101,12 +101,23 @@ int mlc_plan_set(mlc_plan* plan, int index, mlc_fn fn, uint32_t grid, uint32_t b
                  uint32_t lds_bytes, const void* kernarg, size_t size);
 /* Launch entries [begin, end) in order on `stream`. */
 int mlc_plan_run(mlc_plan* plan, int begin, int end, void* stream);
+/* Entry `index` reads the caller's input `input` through the pointer at byte
+ * `offset` of its arguments. */
+int mlc_plan_input(mlc_plan* plan, int index, uint32_t offset, int input);
+/* Launch entries [begin, end) with those pointers replaced by `inputs`. The
+ * plan itself is not changed, so calls may come from several threads. */
+int mlc_plan_call(mlc_plan* plan, int begin, int end, const void* const* inputs, int n_inputs,
+                  void* stream);
 int mlc_plan_destroy(mlc_plan* plan);
 
 /* Stream capture into the context's graph (thread-local capture mode). */
 int mlc_graph_begin(mlc_ctx* ctx, void* stream);
 int mlc_graph_end(mlc_ctx* ctx);
 int mlc_graph_replay(mlc_ctx* ctx, void* stream);
+/* `n` (at most 8) device-to-device copies of 16-byte aligned buffers as one
+ * launch, then the captured graph. */
+int mlc_graph_call(mlc_ctx* ctx, int n, void* const* dst, const void* const* src,
+                   const size_t* bytes, void* stream);
 /* Number of nodes in the captured graph (for checks), or negative. */
 int mlc_graph_node_count(mlc_ctx* ctx, size_t* out);
 
@@ -114,16 +125,16 @@ int mlc_graph_node_count(mlc_ctx* ctx, size_t* out);
  * on `stream`, measured with hipEvents recorded on that stream. */
 int mlc_time_entry(mlc_plan* plan, int index, int iters, void* stream, float* ms_out);
 
-/* The context's invalid-input word (16 bytes of device memory, zeroed when
- * first requested, with a pinned host mirror). Kernels that meet an invalid
+/* The context's invalid-input word (16 bytes of coherent host memory, zeroed
+ * when first requested), by its device address. Kernels that meet an invalid
  * input (an embedding id outside its table) store a non-zero value in it. */
 int mlc_error_word(mlc_ctx* ctx, void** device_word);
-/* Enqueue an asynchronous copy of the word to its host mirror on `stream`
- * (may be captured into a graph). */
+/* Nothing to do since the word is host memory; kept for callers that enqueue
+ * it after a run. */
 int mlc_error_fetch(mlc_ctx* ctx, void* stream);
-/* The host mirror's first int as of the last completed fetch; no sync. */
+/* The word as completed kernels left it; no sync. */
 int mlc_error_poll(mlc_ctx* ctx, int32_t* value);
-/* Synchronize the device, then zero the word and its mirror. */
+/* Synchronize the device, then zero the word. */
 int mlc_error_clear(mlc_ctx* ctx);
 
 /* Synchronize the context's device. */

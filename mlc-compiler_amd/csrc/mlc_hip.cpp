@@ -13,6 +13,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "mlc_hip.h"
@@ -111,6 +112,8 @@ struct Entry {
   uint32_t block = 0;
   uint32_t lds = 0;
   std::vector<unsigned char> args;
+  // (byte offset in args, caller's input) of the pointers mlc_plan_call replaces
+  std::vector<std::pair<uint32_t, int>> inputs;
 };
 
 int launch_raw(hipFunction_t fn, uint32_t grid, uint32_t block, uint32_t lds, const void* args,
@@ -121,6 +124,38 @@ int launch_raw(hipFunction_t fn, uint32_t grid, uint32_t block, uint32_t lds, co
   hipError_t e = hipModuleLaunchKernel(fn, grid, 1, 1, block, 1, 1, lds, stream, nullptr, cfg);
   if (e != hipSuccess) return hip_fail(e, "hipModuleLaunchKernel");
   return MLC_OK;
+}
+
+// ---- every input of a captured pass in one launch (mlc_graph_call)
+//
+// A pass costs the host one launch however many inputs it has, where a
+// memcpy each cost 5 us. Blocks of 16 KiB, 16 bytes a lane and access.
+constexpr int kMaxCopies = 8;
+constexpr uint32_t kCopyBlock = 256, kCopyUnroll = 4;
+constexpr size_t kCopyChunk = size_t{16} * kCopyBlock * kCopyUnroll;
+struct Copies {
+  const char* src[kMaxCopies];
+  char* dst[kMaxCopies];
+  size_t bytes[kMaxCopies];
+  uint32_t end[kMaxCopies];  // one past the last block of each
+};
+
+__global__ void __launch_bounds__(kCopyBlock) copy_inputs(Copies c) {
+  int k = 0;
+  while (blockIdx.x >= c.end[k]) ++k;  // the grid is c.end[last]
+  const size_t first = (size_t)(blockIdx.x - (k == 0 ? 0 : c.end[k - 1])) * kCopyChunk;
+  const char* src = c.src[k];
+  char* dst = c.dst[k];
+  const size_t bytes = c.bytes[k];
+#pragma unroll
+  for (uint32_t u = 0; u < kCopyUnroll; ++u) {
+    const size_t at = first + ((size_t)u * kCopyBlock + threadIdx.x) * 16;
+    if (at + 16 <= bytes) {
+      *reinterpret_cast<uint4*>(dst + at) = *reinterpret_cast<const uint4*>(src + at);
+    } else {
+      for (size_t i = at; i < bytes && i < at + 16; ++i) dst[i] = src[i];
+    }
+  }
 }
 
 // ---- the arena for callers that cannot allocate (mlc_slab_static)
@@ -162,8 +197,8 @@ struct mlc_ctx {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   hipStream_t capturing = nullptr;
-  // invalid-input word: set by kernels on the device, mirrored into pinned
-  // host memory by an asynchronous copy the caller enqueues after its work
+  // invalid-input word: coherent host memory that kernels write by its device
+  // address (only when they meet an invalid input), so a pass copies nothing
   int32_t* err_dev = nullptr;
   volatile int32_t* err_host = nullptr;
 };
@@ -204,7 +239,6 @@ int mlc_ctx_destroy(mlc_ctx* ctx) {
   if (ctx->exec != nullptr) (void)hipGraphExecDestroy(ctx->exec);
   if (ctx->graph != nullptr) (void)hipGraphDestroy(ctx->graph);
   slab_release(ctx->slab);
-  if (ctx->err_dev != nullptr) (void)hipFree(ctx->err_dev);
   if (ctx->err_host != nullptr) (void)hipHostFree(const_cast<int32_t*>(ctx->err_host));
   delete ctx;
   return MLC_OK;
@@ -373,6 +407,46 @@ int mlc_plan_run(mlc_plan* plan, int begin, int end, void* stream) {
   return MLC_OK;
 }
 
+int mlc_plan_input(mlc_plan* plan, int index, uint32_t offset, int input) {
+  if (plan == nullptr || input < 0) return fail(MLC_E_ARG, "mlc_plan_input: bad argument");
+  if (index < 0 || static_cast<size_t>(index) >= plan->entries.size())
+    return fail(MLC_E_RANGE, "mlc_plan_input: index out of range");
+  Entry& e = plan->entries[static_cast<size_t>(index)];
+  if (offset % sizeof(void*) != 0 || offset + sizeof(void*) > e.args.size())
+    return fail(MLC_E_RANGE, "mlc_plan_input: offset outside the entry's arguments");
+  e.inputs.emplace_back(offset, input);
+  return MLC_OK;
+}
+
+int mlc_plan_call(mlc_plan* plan, int begin, int end, const void* const* inputs, int n_inputs,
+                  void* stream) {
+  if (plan == nullptr || n_inputs < 0 || (inputs == nullptr && n_inputs > 0))
+    return fail(MLC_E_ARG, "mlc_plan_call: bad argument");
+  if (begin < 0 || end < begin || static_cast<size_t>(end) > plan->entries.size())
+    return fail(MLC_E_RANGE, "mlc_plan_call: range out of bounds");
+  // the plan stays as it is: concurrent calls each patch a copy of their own
+  unsigned char args[1024];
+  for (int i = begin; i < end; ++i) {
+    const Entry& e = plan->entries[static_cast<size_t>(i)];
+    if (e.fn == nullptr) return fail(MLC_E_STATE, "mlc_plan_call: entry was never set");
+    const unsigned char* at = e.args.data();
+    if (!e.inputs.empty()) {
+      if (e.args.size() > sizeof(args))
+        return fail(MLC_E_RANGE, "mlc_plan_call: an entry's arguments are too long to patch");
+      std::memcpy(args, e.args.data(), e.args.size());
+      for (const auto& p : e.inputs) {
+        if (p.second >= n_inputs) return fail(MLC_E_RANGE, "mlc_plan_call: too few inputs");
+        std::memcpy(args + p.first, &inputs[p.second], sizeof(void*));
+      }
+      at = args;
+    }
+    int rc = launch_raw(e.fn, e.grid, e.block, e.lds, at, e.args.size(),
+                        static_cast<hipStream_t>(stream));
+    if (rc != MLC_OK) return rc;
+  }
+  return MLC_OK;
+}
+
 int mlc_plan_destroy(mlc_plan* plan) {
   delete plan;
   return MLC_OK;
@@ -412,6 +486,34 @@ int mlc_graph_replay(mlc_ctx* ctx, void* stream) {
   if (ctx->exec == nullptr) return fail(MLC_E_STATE, "mlc_graph_replay: nothing captured");
   MLC_HIP(hipGraphLaunch(ctx->exec, static_cast<hipStream_t>(stream)));
   return MLC_OK;
+}
+
+int mlc_graph_call(mlc_ctx* ctx, int n, void* const* dst, const void* const* src,
+                   const size_t* bytes, void* stream) {
+  if (ctx == nullptr || n < 0 || n > kMaxCopies || (n > 0 && (dst == nullptr || src == nullptr ||
+                                                             bytes == nullptr)))
+    return fail(MLC_E_ARG, "mlc_graph_call: bad argument");
+  Copies c = {};
+  uint32_t blocks = 0;
+  int used = 0;
+  for (int i = 0; i < n; ++i) {
+    if (bytes[i] == 0 || dst[i] == src[i]) continue;
+    if (reinterpret_cast<uintptr_t>(dst[i]) % 16 != 0 || reinterpret_cast<uintptr_t>(src[i]) % 16 != 0)
+      return fail(MLC_E_ARG, "mlc_graph_call: a copy is not 16-byte aligned");
+    const size_t need = (bytes[i] + kCopyChunk - 1) / kCopyChunk;
+    if (need > 0x7fffffffu - blocks) return fail(MLC_E_RANGE, "mlc_graph_call: copy too large");
+    c.src[used] = static_cast<const char*>(src[i]);
+    c.dst[used] = static_cast<char*>(dst[i]);
+    c.bytes[used] = bytes[i];
+    blocks += static_cast<uint32_t>(need);
+    c.end[used++] = blocks;
+  }
+  if (blocks != 0) {
+    hipLaunchKernelGGL(copy_inputs, dim3(blocks), dim3(kCopyBlock), 0,
+                       static_cast<hipStream_t>(stream), c);
+    MLC_HIP(hipGetLastError());
+  }
+  return mlc_graph_replay(ctx, stream);
 }
 
 int mlc_graph_node_count(mlc_ctx* ctx, size_t* out) {
@@ -458,14 +560,12 @@ int mlc_error_word(mlc_ctx* ctx, void** device_word) {
   if (ctx == nullptr || device_word == nullptr) return fail(MLC_E_ARG, "mlc_error_word: bad argument");
   if (ctx->err_dev == nullptr) {
     MLC_HIP(hipSetDevice(ctx->device));
-    void* d = nullptr;
     void* h = nullptr;
-    MLC_HIP(hipMalloc(&d, kErrorWordBytes));
-    hipError_t e = hipHostMalloc(&h, kErrorWordBytes, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipMemset(d, 0, kErrorWordBytes);
+    void* d = nullptr;
+    MLC_HIP(hipHostMalloc(&h, kErrorWordBytes, hipHostMallocMapped | hipHostMallocCoherent));
+    hipError_t e = hipHostGetDevicePointer(&d, h, 0);
     if (e != hipSuccess) {
-      (void)hipFree(d);
-      if (h != nullptr) (void)hipHostFree(h);
+      (void)hipHostFree(h);
       return hip_fail(e, "mlc_error_word");
     }
     std::memset(h, 0, kErrorWordBytes);
@@ -479,8 +579,7 @@ int mlc_error_word(mlc_ctx* ctx, void** device_word) {
 int mlc_error_fetch(mlc_ctx* ctx, void* stream) {
   if (ctx == nullptr) return fail(MLC_E_ARG, "mlc_error_fetch: null ctx");
   if (ctx->err_dev == nullptr) return fail(MLC_E_STATE, "mlc_error_fetch: no error word");
-  MLC_HIP(hipMemcpyAsync(const_cast<int32_t*>(ctx->err_host), ctx->err_dev, kErrorWordBytes,
-                         hipMemcpyDeviceToHost, static_cast<hipStream_t>(stream)));
+  (void)stream;  // the word is host memory that kernels write: nothing to copy
   return MLC_OK;
 }
 
@@ -495,7 +594,6 @@ int mlc_error_clear(mlc_ctx* ctx) {
   if (ctx->err_dev == nullptr) return MLC_OK;
   MLC_HIP(hipSetDevice(ctx->device));
   MLC_HIP(hipDeviceSynchronize());
-  MLC_HIP(hipMemset(ctx->err_dev, 0, kErrorWordBytes));
   for (size_t i = 0; i < kErrorWordBytes / sizeof(int32_t); ++i) ctx->err_host[i] = 0;
   return MLC_OK;
 }

@@ -3,7 +3,8 @@
 Calling a :class:`CompiledModel` copies the inputs into fixed device
 buffers and replays one captured hipGraph of the whole schedule (generated
 kernels through ``libmlc_hip.so``, library calls through torch), then hands
-back views of the output buffers.
+back views of the output buffers. A short schedule is launched kernel by
+kernel on the caller's inputs instead (``_launch_directly``).
 
 Memory (``_Buffers``):
 
@@ -11,7 +12,9 @@ Memory (``_Buffers``):
 * planned intermediates are slices of the arena -- one ``hipMalloc`` slab, or
   the library's static array -- at the planner's offsets, so every pointer a
   kernel sees is the same on every call (what makes capture valid);
-* inputs are copied into buffers of their own each call, never aliased;
+* inputs are read where the caller has them when a pass is launched kernel by
+  kernel, and copied into buffers of their own in front of a graph; nothing
+  aliases one after the call's work is done;
 * outputs alias storage the next call overwrites (clone to keep one).
 
 With ``memory_planning`` off the plan is "eager": intermediates are allocated
@@ -44,6 +47,10 @@ import torch
 from ..config import Config
 from ..ir.graph import Graph, Value
 from ..kernels import ExternKernel, Schedule
+
+
+#: launches of a pass above which it is always a graph
+MAX_DIRECT = 32
 
 
 class ExecutionError(Exception):
@@ -289,6 +296,10 @@ class CompiledModel:
         self._buffers = _Buffers(self)
         self._plan: list | None = None
         self._runs: list | None = None
+        #: inputs are read in place and the runs launched one by one
+        self._direct = False
+        #: memory of this model that a caller's input may be a view of
+        self._own: list[tuple[int, int]] = []
         self._captured = False
         self._capture_stream = None
         self._static_outputs: Any = None
@@ -352,6 +363,87 @@ class CompiledModel:
                 i += 1
         group = getattr(self._module, "compile_runs", None)
         self._runs = group(launches) if group is not None else launches
+        if (self.cfg.cuda_graphs and self.device.type == "cuda"
+                and hasattr(self._module, "bind_inputs") and self._launch_directly(launches, table)):
+            self._module.bind_inputs(self._runs, {t.data_ptr(): i for i, t in
+                                                  enumerate(self._buffers.inputs)})
+            mine = {id(t) for t in (*self._buffers.inputs, *self.params.values())}
+            held = [t for t in table.values() if id(t) not in mine]
+            self._own = [(t.data_ptr(), t.data_ptr() + t.numel() * t.element_size())
+                         for t in (*held, *([self._arena] if self._arena is not None else []))]
+            self._direct = True
+
+    def _launch_directly(self, launches, table) -> bool:
+        """Whether a pass launches its kernels one by one on the caller's own
+        inputs rather than replaying a graph behind a copy of them.
+
+        A graph costs the host 21 us to launch plus 0.5 a node, and its inputs
+        a copy; a native launch costs 3 us, a library call through torch about
+        9. So one by one wins for a few launches (embeddings b32 s128: 4
+        launches, 42 us as a graph, 18 one by one), and for more while the
+        device has work for longer than the host needs to issue it, where the
+        copy is what is saved. Library calls keep the addresses they were
+        bound with, so none may read an input; no kernel may write one and no
+        output may be one."""
+        names = {v.buffer.name for v in self.graph.inputs}
+        at = {t.data_ptr() for t in self._buffers.inputs if t.numel()}
+        if len(at) != len(self._buffers.inputs):
+            return False
+        writes = [v for k in self.schedule.kernels if k.name not in self._constants
+                  for v in k.writes()]
+        bound = [c for kind, c in launches if kind == "extern" and isinstance(c, ExternCall)]
+        read = [v for k, (_, c) in zip(self.schedule.kernels, self._plan)
+                if any(c is x for x in bound) for v in k.reads()]
+        if any(v.buffer.name in names for v in (*self.graph.outputs, *writes, *read)):
+            return False
+        count = sum(kind != "const" for kind, _ in launches)
+        host = 3.0 * (count - len(bound)) + 9.0 * len(bound)
+        return count <= MAX_DIRECT and host <= max(24.0, self._device_estimate(count))
+
+    def _device_estimate(self, count: int) -> float:
+        """Microseconds the device is busy with a pass, at least: the launches'
+        floor, and their buffers at 5 TB/s."""
+        moved = sum(v.buffer.nbytes for k in self.schedule.kernels if k.name not in self._constants
+                    for v in (*k.reads(), *k.writes()))
+        return 1.5 * count + moved / 5e6
+
+    def _in_place(self, inputs) -> list[int] | None:
+        """Addresses of the caller's inputs, or ``None`` when one of them has to
+        be converted, re-laid, moved or protected: not this dtype, contiguous
+        and 16-byte aligned on this GPU, or a view of memory this pass writes
+        (an output fed back)."""
+        out = []
+        for t, own in zip(inputs, self._buffers.inputs):
+            if type(t) is not torch.Tensor or t.dtype != own.dtype or t.device != own.device \
+                    or not t.is_contiguous() or t.is_neg():
+                return None
+            p = t.data_ptr()
+            end = p + own.numel() * own.element_size()
+            if p % 16 or any(p < hi and lo < end for lo, hi in self._own):
+                return None
+            out.append(p)
+        return out
+
+    def _call_directly(self, inputs, stream: int) -> None:
+        ptrs = self._in_place(inputs)
+        if ptrs is None:
+            for dst, src in zip(self._buffers.inputs, inputs):
+                dst.copy_(src.reshape(-1), non_blocking=True)
+            ptrs = [t.data_ptr() for t in self._buffers.inputs]
+        self._module.call(self._runs, ptrs, stream)
+
+    def _replay(self, inputs, stream: int) -> None:
+        """The inputs into their buffers, then the graph: plain device tensors
+        in one launch with it, others through torch."""
+        copies = []
+        for t, own in zip(inputs, self._buffers.inputs):
+            if (type(t) is torch.Tensor and t.dtype == own.dtype and t.device == own.device
+                    and t.is_contiguous() and not t.is_neg() and t.data_ptr() % 16 == 0
+                    and len(copies) < self._module.MAX_COPIES):
+                copies.append((own.data_ptr(), t.data_ptr(), own.numel() * own.element_size()))
+            else:
+                own.copy_(t.reshape(-1), non_blocking=True)
+        self._module.graph_call(copies, stream)
 
     def run_one(self, k, table: dict[str, torch.Tensor]) -> None:
         if isinstance(k, ExternKernel):
@@ -371,6 +463,10 @@ class CompiledModel:
         else:
             for k in self.schedule.kernels:
                 self.run_one(k, table)
+        self._fetch_errors()
+
+    def _fetch_errors(self) -> None:
+        """For a runner that reports invalid inputs by an enqueued copy."""
         fetch = getattr(self._module, "fetch_errors", None)
         if fetch is not None:
             fetch()
@@ -388,9 +484,7 @@ class CompiledModel:
                 self.run_one(k, table)
                 for name in plan.free_at.get(i, ()):
                     table.pop(name, None)
-            fetch = getattr(self._module, "fetch_errors", None)
-            if fetch is not None:
-                fetch()
+            self._fetch_errors()
             return self._collect(table)
         table = self._buffers.resident(inputs)
         self._resolve(table)
@@ -402,12 +496,22 @@ class CompiledModel:
         if not (self.cfg.cuda_graphs and self.device.type == "cuda"):
             out = self.forward(*inputs)
         else:
-            if not self._captured:
-                self._capture(inputs)
             self._check_inputs(inputs)
-            for dst, src in zip(self._buffers.inputs, inputs):
-                dst.copy_(src.reshape(-1), non_blocking=True)
-            self._module.replay(torch.cuda.current_stream(self.device).cuda_stream)
+            if self._plan is None:
+                self._resolve(self._buffers.resident(inputs))
+            stream = torch.cuda.current_stream(self.device).cuda_stream
+            if self._direct:
+                if self._static_outputs is None:
+                    self._static_outputs = self._collect(self._buffers.table)
+                if torch.cuda.current_device() == self._module.index:
+                    self._call_directly(inputs, stream)
+                else:
+                    with torch.cuda.device(self.device):
+                        self._call_directly(inputs, stream)
+            else:
+                if not self._captured:
+                    self._capture(inputs)
+                self._replay(inputs, stream)
             out = self._static_outputs
         if self.cfg.sync_input_checks:
             self.check_errors()
@@ -462,9 +566,9 @@ class CompiledModel:
     def _raise_pending(self) -> None:
         """Raise for an invalid input (an embedding id outside its table) that
         an earlier, completed call met. The native gather cannot raise where
-        torch's ``aten.embedding`` would, so it flags the id in a device word
-        that every run copies back asynchronously; the flag is cleared before
-        raising, so the call after the exception runs normally."""
+        torch's ``aten.embedding`` would, so it flags the id in a word of host
+        memory; the flag is cleared before raising, so the call after the
+        exception runs normally."""
         poll = getattr(self._module, "pending_error", None)
         msg = poll() if poll is not None else None
         if msg is not None:
@@ -474,10 +578,9 @@ class CompiledModel:
     def check_errors(self) -> None:
         """Wait for every call so far to finish and raise
         :class:`ExecutionError` if one of them met an invalid input."""
-        fetch = getattr(self._module, "fetch_errors", None)
-        if fetch is None:
+        if getattr(self._module, "pending_error", None) is None:
             return
-        fetch()
+        self._fetch_errors()
         if self.device.type == "cuda":
             torch.cuda.synchronize(self.device)
         self._raise_pending()

@@ -17,10 +17,12 @@ the per-model native state the MI355X design adds:
   ``capture_end``, ``replay``);
 * hipEvent timing of one bound kernel in place (``time_bound``);
 * the invalid-input word: the native embedding gather flags an id outside
-  its table there (torch raises ``IndexError`` for one); every run enqueues
-  an asynchronous copy of the word to pinned host memory (``fetch_errors``,
-  captured into the graph too) and ``pending_error`` reads that copy without
-  waiting for the device.
+  its table there (torch raises ``IndexError`` for one). It is coherent host
+  memory, so a pass enqueues nothing for it and ``pending_error`` reads it
+  without waiting for the device;
+* the caller's inputs: read where they are by launches made one by one
+  (``bind_inputs``, ``call``), or copied in by one launch in front of the graph
+  (``graph_call``).
 """
 
 from __future__ import annotations
@@ -96,6 +98,8 @@ class HipRuntime:
                                               {**self.product_table, **self.group_table})):
             self._load(path.read_bytes(), sorted({s.symbol for s in table.values()}))
         self._plans: list[ctypes.c_void_p] = []
+        #: native plan -> its launches, by entry
+        self._launches: dict[int, list[Bound]] = {}
         self._arena_tensor: torch.Tensor | None = None
         self._static_arena = bool(getattr(cfg, "static_arena", False))
         #: device address of the context's invalid-input word, if a kernel
@@ -183,20 +187,10 @@ class HipRuntime:
         """Whether a kernel of this module can flag an invalid input."""
         return self._error_word is not None
 
-    def fetch_errors(self, stream: int | None = None) -> None:
-        """Enqueue the copy of the invalid-input word to its pinned host
-        mirror on ``stream`` (torch's current stream by default). It is
-        issued after a run's kernels, so under capture it becomes the graph's
-        last node."""
-        if self._error_word is not None:
-            native.check(self.lib.mlc_error_fetch(self._ctx, _stream() if stream is None
-                                                  else stream), "mlc_error_fetch")
-
     def pending_error(self) -> str | None:
         """The message for an invalid input flagged by a completed run, read
-        from the host mirror without waiting for the device; ``None`` if no
-        completed run flagged one. Runs still in flight are seen by a later
-        call."""
+        without waiting for the device; ``None`` if no completed run flagged
+        one. Runs still in flight are seen by a later call."""
         if self._error_word is None:
             return None
         value = ctypes.c_int32()
@@ -207,16 +201,15 @@ class HipRuntime:
                 "id); the rows it addressed were written as zeros")
 
     def clear_errors(self) -> None:
-        """Wait for the device, then zero the word and its mirror."""
+        """Wait for the device, then zero the word."""
         if self._error_word is not None:
             native.check(self.lib.mlc_error_clear(self._ctx), "mlc_error_clear")
 
     def check_errors(self) -> None:
-        """Synchronize, fetch the word, and raise :class:`native.NativeError`
-        if any run so far flagged an invalid input (clearing the flag)."""
+        """Synchronize and raise :class:`native.NativeError` if any run so far
+        flagged an invalid input (clearing the flag)."""
         if self._error_word is None:
             return
-        self.fetch_errors()
         torch.cuda.synchronize(self.device)
         msg = self.pending_error()
         if msg is not None:
@@ -253,6 +246,7 @@ class HipRuntime:
         native.check(self.lib.mlc_plan_create(self._ctx, len(kernels), ctypes.byref(handle)),
                      "mlc_plan_create")
         self._plans.append(handle)
+        self._launches[handle.value] = kernels
         for i, b in enumerate(kernels):
             native.check(self.lib.mlc_plan_set(handle, i, b.fn, b.grid, b.block, b.lds, b.args,
                                                len(b.args)), "mlc_plan_set")
@@ -268,6 +262,31 @@ class HipRuntime:
             else:
                 runs.append((kind, payload))
         return runs
+
+    def bind_inputs(self, runs: list, addresses: dict[int, int]) -> None:
+        """Let ``call`` replace the buffers at ``addresses`` (address of an
+        input's own buffer -> the input's position) wherever a launch of
+        ``runs`` reads them."""
+        for kind, payload in runs:
+            if kind != "kernel":
+                continue
+            for i in range(payload.begin, payload.end):
+                args = self._launches[payload.plan][i].args
+                for at, (ptr,) in enumerate(struct.iter_unpack("<Q", args)):
+                    if ptr in addresses:
+                        native.check(self.lib.mlc_plan_input(payload.plan, i, 8 * at,
+                                                             addresses[ptr]), "mlc_plan_input")
+
+    def call(self, runs: list, inputs, stream: int) -> None:
+        """Launch ``runs`` one by one on the given input addresses."""
+        n = len(inputs)
+        ptrs = (ctypes.c_void_p * n)(*inputs)
+        for kind, payload in runs:
+            if kind == "kernel":
+                native.check(self.lib.mlc_plan_call(payload.plan, payload.begin, payload.end, ptrs,
+                                                    n, stream), "mlc_plan_call")
+            elif kind == "extern":
+                payload.run()
 
     # -- arena -----------------------------------------------------------------
     def arena(self, nbytes: int) -> torch.Tensor:
@@ -303,6 +322,18 @@ class HipRuntime:
 
     def replay(self, stream: int) -> None:
         native.check(self.lib.mlc_graph_replay(self._ctx, stream), "mlc_graph_replay")
+
+    #: copies ``graph_call`` takes at once
+    MAX_COPIES = 8
+
+    def graph_call(self, copies: list[tuple[int, int, int]], stream: int) -> None:
+        """``(dst, src, bytes)`` device copies as one launch, then the graph."""
+        n = len(copies)
+        dst, src = (ctypes.c_void_p * n)(), (ctypes.c_void_p * n)()
+        size = (ctypes.c_size_t * n)()
+        for i, (d, s, b) in enumerate(copies):
+            dst[i], src[i], size[i] = d, s, b
+        native.check(self.lib.mlc_graph_call(self._ctx, n, dst, src, size, stream), "mlc_graph_call")
 
     def graph_nodes(self) -> int:
         n = ctypes.c_size_t()

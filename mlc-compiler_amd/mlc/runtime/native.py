@@ -106,10 +106,13 @@ SIGNATURES = {
     "mlc_plan_create": ([_vp, _c_int, _pvp], _c_int),
     "mlc_plan_set": ([_vp, _c_int, _vp, _c_u32, _c_u32, _c_u32, _vp, _c_size], _c_int),
     "mlc_plan_run": ([_vp, _c_int, _c_int, _vp], _c_int),
+    "mlc_plan_input": ([_vp, _c_int, _c_u32, _c_int], _c_int),
+    "mlc_plan_call": ([_vp, _c_int, _c_int, _pvp, _c_int, _vp], _c_int),
     "mlc_plan_destroy": ([_vp], _c_int),
     "mlc_graph_begin": ([_vp, _vp], _c_int),
     "mlc_graph_end": ([_vp], _c_int),
     "mlc_graph_replay": ([_vp, _vp], _c_int),
+    "mlc_graph_call": ([_vp, _c_int, _pvp, _pvp, ctypes.POINTER(_c_size), _vp], _c_int),
     "mlc_graph_node_count": ([_vp, ctypes.POINTER(_c_size)], _c_int),
     "mlc_time_entry": ([_vp, _c_int, _c_int, _vp, ctypes.POINTER(ctypes.c_float)], _c_int),
     "mlc_error_word": ([_vp, _pvp], _c_int),
