@@ -78,6 +78,12 @@ class Operand:
         return (self.k == 1 and self.row % elements == 0 and self.base % elements == 0
                 and (batches == 1 or self.batch % elements == 0))
 
+    def columns_aligned(self, elements: int, batches: int) -> bool:
+        """Rows at unit stride, every k's run of them starting on a multiple
+        of ``elements``."""
+        return (self.k != 1 and self.row == 1 and self.k % elements == 0
+                and self.base % elements == 0 and (batches == 1 or self.batch % elements == 0))
+
 
 @dataclass(frozen=True)
 class Product:
@@ -271,7 +277,8 @@ class _Source:
         if p.form[0] == "tiled":
             return [f"  mlc::gemm_tile<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.b.row}, "
                     f"{', '.join(map(str, p.form[1:]))}>(a, b, mt * {TM}, nt * {TN}, store);", "}"]
-        flags = ", ".join(str(o.aligned(E, p.batches) and p.K % E == 0).lower() for o in (p.a, p.b))
+        flags = ", ".join(str(o.aligned(E, p.batches) or o.columns_aligned(E, p.batches)).lower()
+                          for o in (p.a, p.b))
         return [f"  mlc::gemm_staged<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.a.k}, {p.b.row}, {p.b.k}, "
                 f"{TM}, {TN}, {8 * E}, {flags}>(a, b, mt * {TM}, nt * {TN}, store);", "}"]
 

@@ -221,19 +221,36 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
   }
 }
 
+// 16 bytes or 4 elements at an address aligned to one element: the hardware
+// takes unaligned global accesses, one instruction instead of one an element.
+template <class F, class T> __device__ __forceinline__ F load_unaligned(const T* p) {
+  F f;
+  __builtin_memcpy(&f, p, sizeof(F));
+  return f;
+}
+
 // One operand's TR x BK tile, global to registers to LDS ([row][k], rows
-// padded by 16 bytes). ROWS x K is the operand's extent; along k at unit
-// stride (SK == 1) a lane moves 16 bytes of one row, otherwise (rows at unit
-// stride) eight or four k of one row, neighbouring lanes neighbouring rows.
-// Past the extent: the last row again, zeros along k.
+// padded by 16 bytes). ROWS x K is the operand's extent. Three ways in:
+//  * unit stride along k: a lane moves 16 bytes of one row;
+//  * 16 bits, unit stride along the rows: a lane loads 16 bytes of eight rows
+//    at two neighbouring k and writes eight pairs;
+//  * otherwise a lane gathers 16 bytes along k, neighbouring lanes
+//    neighbouring rows.
+// Past the extent: a valid row again, zeros along k.
 template <class T, int ROWS, int K, int SR, int SK, int TR, int BK, int THREADS, bool ALIGNED>
 struct tile_loader {
   typedef typename mma_type<T>::frag frag;
   static constexpr int E = 16 / sizeof(T), PITCH = BK + E;
-  static constexpr int PIECES = TR * (BK / E), PER = (PIECES + THREADS - 1) / THREADS;
-  frag v[PER];
+  static constexpr bool PAIRS = sizeof(T) == 2 && SK != 1 && SR == 1;
+  static constexpr int LOADS = PAIRS ? 2 : 1;       // fragments a lane holds per piece
+  static constexpr int PIECES = TR * (BK / E) / LOADS, PER = (PIECES + THREADS - 1) / THREADS;
+  union word { frag f; T x[E]; };
+  word v[PER][LOADS];
   __device__ __forceinline__ static void where(int id, int& row, int& k) {
-    if constexpr (SK == 1) {
+    if constexpr (PAIRS) {
+      row = id % (TR / E) * E;
+      k = id / (TR / E) * 2;
+    } else if constexpr (SK == 1) {
       row = id / (BK / E);
       k = id % (BK / E) * E;
     } else {
@@ -248,18 +265,37 @@ struct tile_loader {
       if (PIECES % THREADS != 0 && id >= PIECES) continue;
       int row, k;
       where(id, row, k);
-      row = row0 + row < ROWS ? row0 + row : ROWS - 1;
+      row += row0;
       k += k0;
-      const T* q = p + (int64_t)row * SR + (int64_t)k * SK;
-      if constexpr (SK == 1 && ALIGNED) {
-        v[u] = (K % BK == 0 || k < K) ? load_frag<T>(q) : frag{};
-      } else {
-        union { frag f; T x[E]; } w;
-        w.f = frag{};
+      if constexpr (PAIRS) {
 #pragma unroll
-        for (int i = 0; i < E; ++i)
-          if (K % BK == 0 || k + i < K) w.x[i] = q[(int64_t)i * SK];
-        v[u] = w.f;
+        for (int h = 0; h < 2; ++h) {
+          word w;
+          w.f = frag{};
+          if (K % BK == 0 || k + h < K) {
+            const T* q = p + (int64_t)(k + h) * SK;
+            if (ROWS % TR == 0 || row + E <= ROWS) {
+              w.f = ALIGNED ? load_frag<T>(q + row) : load_unaligned<frag>(q + row);
+            } else {
+#pragma unroll
+              for (int i = 0; i < E; ++i) w.x[i] = q[row + i < ROWS ? row + i : ROWS - 1];
+            }
+          }
+          v[u][h] = w;
+        }
+      } else {
+        row = row < ROWS ? row : ROWS - 1;
+        const T* q = p + (int64_t)row * SR + (int64_t)k * SK;
+        word w;
+        w.f = frag{};
+        if (SK == 1 && (K % BK == 0 || k + E <= K)) {
+          w.f = ALIGNED ? load_frag<T>(q) : load_unaligned<frag>(q);
+        } else {
+#pragma unroll
+          for (int i = 0; i < E; ++i)
+            if (K % BK == 0 || k + i < K) w.x[i] = q[(int64_t)i * SK];
+        }
+        v[u][0] = w;
       }
     }
   }
@@ -270,7 +306,13 @@ struct tile_loader {
       if (PIECES % THREADS != 0 && id >= PIECES) continue;
       int row, k;
       where(id, row, k);
-      *reinterpret_cast<frag*>(&lds[row][k]) = v[u];
+      if constexpr (PAIRS) {
+#pragma unroll
+        for (int i = 0; i < E; ++i)
+          *reinterpret_cast<pack<T, 2>*>(&lds[row + i][k]) = pack<T, 2>{{v[u][0].x[i], v[u][1].x[i]}};
+      } else {
+        *reinterpret_cast<frag*>(&lds[row][k]) = v[u][0].f;
+      }
     }
   }
 };
@@ -332,14 +374,17 @@ template <class T> __device__ __forceinline__ float ld_of(float x) { return x; }
 template <> __device__ __forceinline__ float ld_of<f16>(float x) { return round_f16(x); }
 template <> __device__ __forceinline__ float ld_of<bf16>(float x) { return round_bf16(x); }
 
-// Four consecutive columns of one row, dropped past M and N; 8- or 16-byte
-// stores when every row starts on that boundary.
+// Four consecutive columns of one row, dropped past M and N, in one store
+// except at the end of a row.
 template <class T, int M, int N, int LDC, bool ALIGNED>
 __device__ __forceinline__ void store4(T* __restrict__ c, int m, int n, const float (&v)[4]) {
   if (m >= M || n >= N) return;
   T* p = c + (int64_t)m * LDC + n;
   if constexpr (ALIGNED) {
     store_pack<4>(p, v);
+  } else if (n + 4 <= N) {
+    const pack<T, 4> w = {{cvt<T>(v[0]), cvt<T>(v[1]), cvt<T>(v[2]), cvt<T>(v[3])}};
+    __builtin_memcpy(p, &w, sizeof(w));
   } else {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
