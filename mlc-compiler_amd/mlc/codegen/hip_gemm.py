@@ -16,10 +16,11 @@ rounding.
 
 Measured in graphs of 24-48 products over 12 weights, fp16, library / tiled:
 16x2048x512 (M x N x K) 3.6 / 2.0 us, 128x768x768 4.6 / 2.3, 128x3072x768
-7.8 / 3.7, 128x768x3072 7.6 / 4.8, 512x768x768 7.2 / 3.7, 1182x768x768
-7.9 / 5.2, 2048x2304x768 16.3 / 12.5, 2048x768x3072 18.8 / 18.3; past 10 GFLOP
-the library wins (4096x2304x768 20.1 / 24.0). fp32: 128x3072x768 15.3 / 7.6,
-128x768x3072 12.0 / 9.7, 1024x768x768 14.1 / 12.4, 1024x2304x768 36.4 / 39.
+7.8 / 3.7, 128x768x3072 7.6 / 4.8, 525x768x768 7.3 / 4.0, 2048x2304x768
+16.1 / 10.5, 2048x768x3072 19.0 / 14.9, 4096x3072x768 24.4 / 20.8,
+16384x2304x768 70 / 58 (990 TFLOP/s, of 1340 that a large library product
+reaches here). fp32: 128x3072x768 15.3 / 7.6, 128x768x3072 12.0 / 9.7,
+1024x768x768 13.8 / 12.8.
 """
 
 from __future__ import annotations
@@ -44,23 +45,25 @@ TILES = ((16, 16, 1, 1, (1, 2, 4)), (16, 32, 1, 2, (2, 4)), (16, 32, 1, 1, (3,))
          (32, 32, 2, 2, (1, 2, 4)), (32, 48, 2, 1, (2, 4)), (32, 64, 2, 2, (1, 2)),
          (64, 64, 2, 2, (1, 2)), (64, 96, 2, 2, (1, 2)), (64, 128, 2, 4, (1,)),
          (96, 96, 2, 2, (1,)), (128, 96, 2, 2, (1,)), (128, 128, 2, 4, (1,)),
-         (128, 192, 2, 4, (1,)))
+         (128, 192, 2, 4, (1,)), (128, 256, 2, 4, (1,)), (256, 256, 4, 2, (1,)))
 #: floating-point operations up to which the tiled form is at least the
-#: library's speed (the table above), by element size; and for a square-ish
-#: weight, where it holds on (16384x768x768 fp16: 25.0 us, tiled 23.5)
-TILED_FLOPS = {2: 10e9, 4: 2.2e9}
-NARROW, NARROW_FLOPS = 1024, {2: 20e9, 4: 2.2e9}
-#: the same with pointwise kernels in the epilogue, against the library and
-#: those kernels after it (fp16): 8192x3072x768 + bias + GELU 58 us against
-#: 46 + 19, 16384x3072x768 111 against 74 + 36; the bias and re-layout of
-#: 16384x2304x768 cost 3 us on 68 against 67 + 29; 16384x768x3072 + bias +
-#: residual 85 against 69 + 12. An epilogue with a transcendental is arithmetic
-#: that nothing overlaps once a CU holds one large tile.
-MERGED_FLOPS, MERGED_MATH_FLOPS = 60e9, 40e9
+#: library's speed, by element size: fp16 16384x2304x768 58 us against 70,
+#: 16384x3072x768 76 against 70; with long sums 8192x768x3072 39.6 against
+#: 40.4, 16384x768x3072 70 against 65; fp32 2048x768x768 21 against 27, but
+#: 525x768x3072 30 against 27
+TILED_FLOPS, LONG_K, LONG_K_FLOPS = {2: 60e9, 4: 2.2e9}, 1024, 40e9
+#: past this many columns (a vocabulary head) the weights are most of the
+#: traffic and padded rows cost in full: 512x50257x768 fp16 62 us against 66
+#: and 16 rows 16.0 against 17.8, but 333 rows 58 against 46, 64 rows 20.3
+#: against 19.6, 1024 rows 124 against 117
+WIDE, WIDE_FLOPS = 16384, 40e9
+#: the lines with pointwise kernels in the epilogue, against the library and
+#: those kernels after it: 16384x768x3072 + bias + residual 71 us against
+#: 65 + 12. An epilogue with a transcendental is arithmetic that little
+#: overlaps: 8192x3072x768 + bias + GELU 55 us against 48 + 19, but
+#: 16384x3072x768 104-111 against 70 + 36.
+MERGED_FLOPS, MERGED_MATH_FLOPS = 80e9, 40e9
 TRANSCENDENTAL = {"erf", "exp", "tanh", "sigmoid", "sin", "cos", "log", "pow"}
-#: widest product measured: a vocabulary head streams its weights, where the
-#: library's larger tiles win
-MAX_COLUMNS = 4096
 
 
 @dataclass(frozen=True)
@@ -129,8 +132,12 @@ def tile_cost(M: int, N: int, K: int, batches: int, size: int, tile: tuple) -> f
 
 
 def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None:
-    """The cheapest tile by ``tile_cost``, with the deepest ring that fits LDS
-    (half of it where a CU has more than one tile to do).
+    """The cheapest tile by ``tile_cost``, with the deepest ring that fits LDS.
+
+    In 16 bits, a product of more than one tile per CU takes tiles of at least
+    128 x 128 (smaller ones reload A and B too often: 4096x2304x768 took 21.8 us
+    in 128 x 96, 18.3 in 128 x 192), and a ring of half of LDS: two workgroups
+    at a time, one's epilogue and first loads under the other's products.
 
     In fp32 a k-split of 4 is kept up to 128 rows, where the library sums k in
     as many parts: fewer, longer sums would be further from float64 than it
@@ -140,6 +147,8 @@ def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None
     for TM, TN, WM, WN, splits in TILES:
         if TM > max(16, 2 * M):
             continue
+        crowded = size == 2 and -(-batches * -(-M // TM) * -(-N // TN) // XCDS) > CUS // XCDS
+        small = crowded and TM * TN < 128 * 128
         fewest = 1
         if size == 4:
             fewest = (4 if M <= 128 else 2) if TM * TN <= 32 * 48 else 2 if TM * TN <= 64 * 96 else 1
@@ -152,23 +161,30 @@ def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None
                 return next((n for n in (4, 3, 2)
                              if min(n, steps) * WK * (TM + TN) * 128 <= lds), None)
 
-            # several tiles per CU: two workgroups at a time, one's epilogue
-            # and first loads under the other's products
-            tiles = batches * -(-M // TM) * -(-N // TN)
-            crowded = -(-tiles // XCDS) > CUS // XCDS
             stages = (deepest(LDS_BYTES // 2) if crowded else None) or deepest(LDS_BYTES)
             if stages is None:
                 continue
             tile = (TM, TN, WM, WN, WK, min(stages, max(2, steps)))
-            cost = tile_cost(M, N, K, batches, size, tile)
-            if best is None or cost < best[0]:
-                best = (cost, tile)
+            rank = (small, tile_cost(M, N, K, batches, size, tile))
+            if best is None or rank < best[0]:
+                best = (rank, tile)
     return best[1] if best else None
 
 
 #: staged form: operations up to which it is used, and the rows and columns of
 #: its tile
 STAGED_FLOPS = 2e9
+
+
+def _line(M: int, N: int, K: int, size: int, merged_flops: float) -> float:
+    """Operations up to which a product runs on the tiled form."""
+    if N > WIDE:
+        full = M >= 0.9 * 128 * -(-M // 128)
+        return WIDE_FLOPS if size == 2 and (M <= 32 or full) else 0.0
+    line = TILED_FLOPS[size]
+    if size == 2:
+        line = max(min(line, LONG_K_FLOPS) if K > LONG_K else line, merged_flops)
+    return line
 
 
 def plan_product(k: ExternKernel, merged_flops: float = 0.0) -> Product | None:
@@ -207,10 +223,7 @@ def plan_product(k: ExternKernel, merged_flops: float = 0.0) -> Product | None:
     size = itemsize(x.dtype)
     flops = 2.0 * batches * M * N * K
     E = 16 // size
-    line = (NARROW_FLOPS if max(N, K) <= NARROW else TILED_FLOPS)[size]
-    if size == 2:
-        line = max(line, merged_flops)
-    if (K * size % 128 == 0 and N <= MAX_COLUMNS and flops <= line
+    if (K * size % 128 == 0 and flops <= _line(M, N, K, size, merged_flops)
             and a.aligned(E, batches) and b.aligned(E, batches)):
         tile = choose_tile(M, N, K, batches, size)
         if tile is not None:
@@ -271,12 +284,13 @@ class _Source:
         """``name`` at this batch's first element."""
         return f"  {name} += (int64_t)z * {o.batch if self.p.batches > 1 else 0} + {o.base};"
 
-    def tail(self) -> list[str]:
+    def tail(self, transposed: str = "false", store_t: str = "store") -> list[str]:
         p, T = self.p, self.storage
         (TM, TN), E = self.tile, 16 // itemsize(p.a.value.dtype)
         if p.form[0] == "tiled":
             return [f"  mlc::gemm_tile<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.b.row}, "
-                    f"{', '.join(map(str, p.form[1:]))}>(a, b, mt * {TM}, nt * {TN}, store);", "}"]
+                    f"{', '.join(map(str, p.form[1:]))}>(a, b, mt * {TM}, nt * {TN}, store, "
+                    f"{transposed}, {store_t});", "}"]
         flags = ", ".join(str(o.aligned(E, p.batches) or o.columns_aligned(E, p.batches)).lower()
                           for o in (p.a, p.b))
         return [f"  mlc::gemm_staged<{T}, {p.M}, {p.N}, {p.K}, {p.a.row}, {p.a.k}, {p.b.row}, {p.b.k}, "
@@ -342,30 +356,48 @@ def _place(terms, var: str) -> str:
     return " + ".join(parts) or "0u"
 
 
-def _part_lines(part, i: int, N: int, TN: int) -> list[str]:
-    """One pointwise kernel's work on four consecutive columns ``n`` of row
-    ``m``: ``x`` holds the product, already rounded to its storage type.
-    Where its columns are whole tiles, which kernel applies is one scalar
+def _transposed(part, p: Product) -> bool:
+    """Whether a part's stores run along the rows of whole tiles (a per-head V
+    transposed for the attention): four rows of a column go out together."""
+    TM, TN, WK = p.form[1], p.form[2], p.form[5]
+    inner = next((t for t in part.m_terms if t[1] == 1), (1, 1, 0))
+    others = [t for t in (*part.m_terms, *part.n_terms) if t is not inner]
+    return (WK == 1 and p.M % 4 == 0 and inner[2] == 1 and inner[0] % 4 == 0
+            and all(t[2] % 4 == 0 for t in others) and _whole_tiles(part, TN, p.N))
+
+
+def _whole_tiles(part, TN: int, N: int) -> bool:
+    return part.lo % TN == 0 and (part.hi % TN == 0 or part.hi == N)
+
+
+def _in_part(part, N: int, TN: int) -> str:
+    """The test for a part's columns: where they are whole tiles, one scalar
     branch per workgroup."""
+    if part.lo == 0 and part.hi == N:
+        return "true"
+    if _whole_tiles(part, TN, N):
+        return f"nt >= {part.lo // TN} && nt < {-(-part.hi // TN)}"
+    return f"n >= {part.lo} && n < {part.hi}"
+
+
+def _part_lines(part, i: int, N: int, TN: int, along_m: bool = False) -> list[str]:
+    """One pointwise kernel's work on four consecutive columns of row ``m`` from
+    ``n`` (four consecutive rows of column ``n`` from ``m``): ``x`` holds the
+    product, already rounded to its storage type."""
     k = part.kernel
     out = k.outputs[0]
-    if part.lo == 0 and part.hi == N:
-        test = "true"
-    elif part.lo % TN == 0 and part.hi % TN == 0:
-        test = f"nt >= {part.lo // TN} && nt < {part.hi // TN}"
-    else:
-        test = f"n >= {part.lo} && n < {part.hi}"
-    L = [f"    if ({test}) {{", f"      const uint32_t q = n - {part.lo}, row = m;"]
+    L = [f"    if ({_in_part(part, N, TN)}) {{", f"      const uint32_t q = n - {part.lo}, row = m;"]
     names: list[str] = []
     for slot, (a, read) in enumerate(zip(k.inputs, part.reads)):
         if read is None:
             names.append("x[j]")
             continue
+        step = read.row if along_m else read.col
         at = f"p{i}_{slot} + (row * {read.row}u + {read.base}u" + (" + q)" if read.col else ")")
-        if read.col:
-            packed = read.row % 4 == 0 and read.base % 4 == 0
+        if step:
+            packed = step == 1 and read.row % 4 == 0 and read.base % 4 == 0
             L.append(f"      float v{slot}[4];" + (f" mlc::load_pack<4>(v{slot}, {at});" if packed else
-                     f" for (int j = 0; j < 4; ++j) v{slot}[j] = mlc::ld({at} + j);"))
+                     f" for (int j = 0; j < 4; ++j) v{slot}[j] = mlc::ld({at} + j * {step});"))
             names.append(f"v{slot}[j]")
         else:
             L.append(f"      const float v{slot} = mlc::ld({at});")
@@ -380,7 +412,8 @@ def _part_lines(part, i: int, N: int, TN: int) -> list[str]:
     code, _ = r.store(k.out_expr[out.value.name], out.dtype == torch.float16)
     inner = next((t for t in part.n_terms if t[1] == 1), (1, 1, 1))
     terms = (*part.m_terms, *part.n_terms)
-    packed = inner[2] == 1 and all(t is inner or t[2] % 4 == 0 for t in terms) and inner[0] % 4 == 0
+    packed = along_m or (inner[2] == 1 and inner[0] % 4 == 0
+                         and all(t is inner or t[2] % 4 == 0 for t in terms))
     L += [f"        o[j] = {code};", "      }",
           f"      {STORAGE[out.dtype]}* w = o{i} + (({_place(part.m_terms, 'row')}) "
           f"+ ({_place(part.n_terms, 'q')}));"]
@@ -406,10 +439,27 @@ def emit_group(k: ExternKernel, parts) -> tuple[str, LaunchSpec]:
         out = part.kernel.outputs[0]
         params.append(f"{STORAGE[out.dtype]}* __restrict__ o{i}")
         values.append(out.value)
-    L = src.head(params) + ["  auto store = [&](int m, int n, mlc::float4v s) {"]
-    if p.M % src.tile[0] or p.N % src.tile[1]:
-        L.append(f"    if (m >= {p.M} || n >= {p.N}) return;")
-    L.append("    const float x[4] = {" + ", ".join(f"mlc::ld_of<{T}>(s[{j}])" for j in range(4)) + "};")
-    for i, part in enumerate(parts):
-        L += _part_lines(part, i, p.N, src.tile[1])
-    return "\n".join(L + ["  };"] + src.tail()), src.spec("gemm+pointwise", values)
+    L = src.head(params)
+    turned = {i for i, part in enumerate(parts) if p.form[0] == "tiled" and _transposed(part, p)}
+
+    def epilogue(name: str, which, along_m: bool) -> list[str]:
+        lines = [f"  auto {name} = [&](int m, int n, mlc::float4v s) {{"]
+        if p.M % src.tile[0] or p.N % src.tile[1]:
+            lines.append(f"    if (m >= {p.M} || n >= {p.N}) return;")
+        lines.append("    const float x[4] = {"
+                     + ", ".join(f"mlc::ld_of<{T}>(s[{j}])" for j in range(4)) + "};")
+        for i, part in enumerate(parts):
+            if i in which:
+                lines += _part_lines(part, i, p.N, src.tile[1], along_m)
+        return lines + ["  };"]
+
+    # a workgroup whose columns belong to turned parts alone stores along m
+    mixed = [i for i in range(len(parts)) if i not in turned]
+    clear = all(parts[i].hi <= parts[t].lo or parts[i].lo >= parts[t].hi
+                for i in mixed for t in turned)
+    if not turned or not clear:
+        L += epilogue("store", range(len(parts)), False)
+        return "\n".join(L + src.tail()), src.spec("gemm+pointwise", values)
+    L += epilogue("store", mixed, False) + epilogue("store_t", turned, True)
+    test = " || ".join(f"({_in_part(parts[t], p.N, src.tile[1])})" for t in sorted(turned))
+    return "\n".join(L + src.tail(test, "store_t")), src.spec("gemm+pointwise", values)

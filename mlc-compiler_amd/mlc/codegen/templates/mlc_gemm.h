@@ -73,11 +73,13 @@ template <int N> __device__ __forceinline__ void wait_vm() {
 // is written in lane order), so 16 lanes reading one slot of 16 rows hit 64
 // distinct banks.
 //
-// Rows past M or N are read from the last row and dropped by the epilogue.
+// Rows past M or N are read from the last row and dropped by the epilogue:
+// epi(m, n, four columns of a row), or where ``transposed`` (the same for the
+// whole workgroup; without a k-split) epi_t(m, n, four rows of a column).
 template <class T, int M, int N, int K, int LDA, int LDB, int TM, int TN, int WM, int WN, int WK,
-          int NST, class Epi>
+          int NST, class Epi, class EpiT>
 __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __restrict__ b,
-                                          int m0, int n0, Epi epi) {
+                                          int m0, int n0, Epi epi, bool transposed, EpiT epi_t) {
   typedef typename mma_type<T>::frag frag;
   constexpr int PIECE = 128, BK = PIECE / sizeof(T);     // bytes and elements of k per stage
   constexpr int SLOTS = PIECE / 16, RPL = 64 / SLOTS;  // rows per load instruction
@@ -90,7 +92,9 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
   constexpr int RING = IT < NST ? IT : NST;
   constexpr int STAGE = ROWS * PIECE;
   constexpr int PART = WK > 1 ? WK * TM * (TN + 4) * 4 : 0;
-  constexpr int LDS = WK * RING * STAGE > PART ? WK * RING * STAGE : PART;
+  constexpr int TW = TN / WN, RP = TW + 4, ROWBUF = 16 * RP;   // floats of a wave's row buffer
+  constexpr int EPI = WK > 1 ? PART : GW * ROWBUF * 4;
+  constexpr int LDS = WK * RING * STAGE > EPI ? WK * RING * STAGE : EPI;
   __shared__ __attribute__((aligned(1024))) char lds[LDS];
 
   const int lane = threadIdx.x & 63;
@@ -195,11 +199,40 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
   }
 
   if constexpr (WK == 1) {
+    // 16 rows at a time through the wave's own LDS, so that neighbouring lanes
+    // store neighbouring pieces of a row (or, transposed, of a column). From
+    // the accumulators a store covers 32 bytes of each of 16 rows:
+    // 16384x2304x768 fp16 took 68 us so, 59 this way; 128x50257x768, whose
+    // rows are odd, 26 and 23.
+    float* rows = reinterpret_cast<float*>(lds) + w * ROWBUF;
+    __syncthreads();  // the ring is read out
 #pragma unroll
-    for (int i = 0; i < RA; ++i)
+    for (int i = 0; i < RA; ++i) {
+      const int mb = m0 + wm * (TM / WM) + 16 * i, nb = n0 + wn * TW;
 #pragma unroll
       for (int j = 0; j < RB; ++j)
-        epi(m0 + wm * (TM / WM) + 16 * i + r, n0 + wn * (TN / WN) + 16 * j + 4 * g, acc[i][j]);
+        *reinterpret_cast<float4v*>(rows + r * RP + 16 * j + 4 * g) = acc[i][j];
+      __builtin_amdgcn_wave_barrier();
+      if (!transposed) {
+#pragma unroll
+        for (int q0 = 0; q0 < 4 * TW; q0 += 64) {
+          const int q = q0 + lane;
+          if (4 * TW % 64 != 0 && q >= 4 * TW) continue;
+          const int m = q / (TW / 4), n = q % (TW / 4) * 4;
+          epi(mb + m, nb + n, *reinterpret_cast<const float4v*>(rows + m * RP + n));
+        }
+      } else {
+#pragma unroll
+        for (int q0 = 0; q0 < 4 * TW; q0 += 64) {
+          const int q = q0 + lane;
+          if (4 * TW % 64 != 0 && q >= 4 * TW) continue;
+          const int m = q % 4 * 4, n = q / 4;
+          const float* c = rows + m * RP + n;
+          epi_t(mb + m, nb + n, float4v{c[0], c[RP], c[2 * RP], c[3 * RP]});
+        }
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
   } else {
     constexpr int P = TN + 4;
     float* part = reinterpret_cast<float*>(lds);

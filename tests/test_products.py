@@ -51,8 +51,13 @@ def test_which_calls_run_natively():
 
     assert _form(Linear(), half(128, 768), half(768, 768)) == "tiled"
     assert _form(Linear(), half(1, 64), half(48, 64)) == "tiled"
+    assert _form(Linear(), half(16384, 768), half(2304, 768)) == "tiled"
     assert _form(Linear(), half(16384, 768), half(3072, 768)) is None      # past the flops line
-    assert _form(Linear(), half(128, 768), half(50257, 768)) is None       # a vocabulary head
+    assert _form(Linear(), half(16384, 3072), half(768, 3072)) is None     # with long sums
+    # a vocabulary head: few rows, or whole tiles of them
+    for rows, native in ((16, True), (64, False), (128, True), (333, False), (512, True)):
+        assert _form(Linear(), half(rows, 768), half(50257, 768)) == ("tiled" if native else None)
+    assert _form(Linear(), torch.zeros(128, 768), torch.zeros(50257, 768)) is None
     assert _form(Linear(), half(128, 100), half(96, 100)) is None          # k not in whole pieces
     assert _form(Linear(), torch.zeros(64, 64, dtype=torch.float64),
                  torch.zeros(64, 64, dtype=torch.float64)) is None
