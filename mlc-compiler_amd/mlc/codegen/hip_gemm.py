@@ -139,13 +139,17 @@ def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None
     in 128 x 96, 18.3 in 128 x 192), and a ring of half of LDS: two workgroups
     at a time, one's epilogue and first loads under the other's products.
 
+    A large tile over a long sum takes eight waves: four, one a SIMD, leave its
+    LDS reads uncovered (4096x768x3072 took 36 us in a layer in 128 x 96 by four
+    waves, 27 in 128 x 128 by eight).
+
     In fp32 a k-split of 4 is kept up to 128 rows, where the library sums k in
     as many parts: fewer, longer sums would be further from float64 than it
     is (5.0e-7 relative against 2.5e-7 at K = 768)."""
     pieces = K * size // 128
     best = None
     for TM, TN, WM, WN, splits in TILES:
-        if TM > max(16, 2 * M):
+        if TM > max(16, 2 * M) or (K > LONG_K and TM * TN >= 128 * 96 and WM * WN < 8):
             continue
         crowded = size == 2 and -(-batches * -(-M // TM) * -(-N // TN) // XCDS) > CUS // XCDS
         small = crowded and TM * TN < 128 * 128
