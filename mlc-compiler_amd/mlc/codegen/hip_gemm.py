@@ -57,12 +57,11 @@ TILED_FLOPS, LONG_K, LONG_K_FLOPS = {2: 60e9, 4: 2.2e9}, 1024, 40e9
 #: and 16 rows 16.0 against 17.8, but 333 rows 58 against 46, 64 rows 20.3
 #: against 19.6, 1024 rows 124 against 117
 WIDE, WIDE_FLOPS = 16384, 40e9
-#: the lines with pointwise kernels in the epilogue, against the library and
-#: those kernels after it: 16384x768x3072 + bias + residual 71 us against
-#: 65 + 12. An epilogue with a transcendental is arithmetic that little
-#: overlaps: 8192x3072x768 + bias + GELU 55 us against 48 + 19, but
-#: 16384x3072x768 104-111 against 70 + 36.
-MERGED_FLOPS, MERGED_MATH_FLOPS = 80e9, 40e9
+#: the line with pointwise kernels in the epilogue, against the library and
+#: those kernels after it: 16384x3072x768 + bias + GELU 114 us in a layer
+#: against 84 + 38; with long sums 16384x768x3072 + bias + residual 90 against
+#: 73 + 12, 8192 rows 41 against 40 + 8
+MERGED_FLOPS, MERGED_LONG_K_FLOPS = 80e9, 60e9
 TRANSCENDENTAL = {"erf", "exp", "tanh", "sigmoid", "sin", "cos", "log", "pow"}
 
 
@@ -131,7 +130,8 @@ def tile_cost(M: int, N: int, K: int, batches: int, size: int, tile: tuple) -> f
                                            + 5.66e-6 * loads + 6e-6 * TM * TN))
 
 
-def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None:
+def choose_tile(M: int, N: int, K: int, batches: int, size: int,
+                math: bool = False) -> tuple | None:
     """The cheapest tile by ``tile_cost``, with the deepest ring that fits LDS.
 
     In 16 bits, a product of more than one tile per CU takes tiles of at least
@@ -142,6 +142,10 @@ def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None
     A large tile over a long sum takes eight waves: four, one a SIMD, leave its
     LDS reads uncovered (4096x768x3072 took 36 us in a layer in 128 x 96 by four
     waves, 27 in 128 x 128 by eight).
+
+    ``math``: an epilogue with a transcendental. No tile then takes more than
+    half of LDS, so that its arithmetic runs beside another tile's products
+    (16384x3072x768 + GELU 104 us in 128 x 192, 111 in 256 x 256).
 
     In fp32 a k-split of 4 is kept up to 128 rows, where the library sums k in
     as many parts: fewer, longer sums would be further from float64 than it
@@ -166,7 +170,7 @@ def choose_tile(M: int, N: int, K: int, batches: int, size: int) -> tuple | None
                              if min(n, steps) * WK * (TM + TN) * 128 <= lds), None)
 
             stages = (deepest(LDS_BYTES // 2) if crowded else None) or deepest(LDS_BYTES)
-            if stages is None:
+            if stages is None or (math and crowded and deepest(LDS_BYTES // 2) is None):
                 continue
             tile = (TM, TN, WM, WN, WK, min(stages, max(2, steps)))
             rank = (small, tile_cost(M, N, K, batches, size, tile))
@@ -191,7 +195,7 @@ def _line(M: int, N: int, K: int, size: int, merged_flops: float) -> float:
     return line
 
 
-def plan_product(k: ExternKernel, merged_flops: float = 0.0) -> Product | None:
+def plan_product(k: ExternKernel, merged_flops: float = 0.0, math: bool = False) -> Product | None:
     """How a library call's product runs natively, or ``None`` to leave it to
     the library. ``merged_flops``: the line where pointwise kernels run in its
     epilogue, which pays for itself where the product alone does not."""
@@ -229,7 +233,7 @@ def plan_product(k: ExternKernel, merged_flops: float = 0.0) -> Product | None:
     E = 16 // size
     if (K * size % 128 == 0 and flops <= _line(M, N, K, size, merged_flops)
             and a.aligned(E, batches) and b.aligned(E, batches)):
-        tile = choose_tile(M, N, K, batches, size)
+        tile = choose_tile(M, N, K, batches, size, math)
         if tile is not None:
             return Product(batches, M, N, K, a, b, c, bias, ("tiled", *tile))
     if rank == 3 and flops <= STAGED_FLOPS:
@@ -344,7 +348,9 @@ def plan_group(k: ExternKernel, parts) -> Product | None:
         return None
     calls = {e.fn for part in parts for _, x in part.kernel.body for e in subexprs(x)
              if isinstance(e, Call)}
-    return plan_product(k, MERGED_MATH_FLOPS if calls & TRANSCENDENTAL else MERGED_FLOPS)
+    K = k.node.args[0].shape[-1]
+    return plan_product(k, MERGED_LONG_K_FLOPS if K > LONG_K else MERGED_FLOPS,
+                        bool(calls & TRANSCENDENTAL))
 
 
 def _place(terms, var: str) -> str:

@@ -95,6 +95,9 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
   constexpr int TW = TN / WN, RP = TW + 4, ROWBUF = 16 * RP;   // floats of a wave's row buffer
   constexpr int EPI = WK > 1 ? PART : GW * ROWBUF * 4;
   constexpr int LDS = WK * RING * STAGE > EPI ? WK * RING * STAGE : EPI;
+  // whether the columns of every wave's tile fit at once (16 rows always do)
+  constexpr bool COLS = GW * TW * (TM / WM + 4) * (int)sizeof(T) <= LDS;
+  static_assert(GW * TW * 20 * (int)sizeof(T) <= LDS || WK > 1, "column buffer");
   __shared__ __attribute__((aligned(1024))) char lds[LDS];
 
   const int lane = threadIdx.x & 63;
@@ -199,39 +202,56 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
   }
 
   if constexpr (WK == 1) {
-    // 16 rows at a time through the wave's own LDS, so that neighbouring lanes
-    // store neighbouring pieces of a row (or, transposed, of a column). From
-    // the accumulators a store covers 32 bytes of each of 16 rows:
-    // 16384x2304x768 fp16 took 68 us so, 59 this way; 128x50257x768, whose
-    // rows are odd, 26 and 23.
-    float* rows = reinterpret_cast<float*>(lds) + w * ROWBUF;
+    // Through the wave's own LDS, so that neighbouring lanes store neighbouring
+    // pieces of a row (or, transposed, of a column). From the accumulators a
+    // store covers 32 bytes of each of 16 rows: 16384x2304x768 fp16 took 68 us
+    // so, 58 this way; 128x50257x768, whose rows are odd, 26 and 23.
+    const int mw = m0 + wm * (TM / WM), nw = n0 + wn * TW;
     __syncthreads();  // the ring is read out
+    if (!transposed) {
+      float* rows = reinterpret_cast<float*>(lds) + w * ROWBUF;
 #pragma unroll
-    for (int i = 0; i < RA; ++i) {
-      const int mb = m0 + wm * (TM / WM) + 16 * i, nb = n0 + wn * TW;
+      for (int i = 0; i < RA; ++i) {
 #pragma unroll
-      for (int j = 0; j < RB; ++j)
-        *reinterpret_cast<float4v*>(rows + r * RP + 16 * j + 4 * g) = acc[i][j];
-      __builtin_amdgcn_wave_barrier();
-      if (!transposed) {
+        for (int j = 0; j < RB; ++j)
+          *reinterpret_cast<float4v*>(rows + r * RP + 16 * j + 4 * g) = acc[i][j];
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
         for (int q0 = 0; q0 < 4 * TW; q0 += 64) {
           const int q = q0 + lane;
           if (4 * TW % 64 != 0 && q >= 4 * TW) continue;
           const int m = q / (TW / 4), n = q % (TW / 4) * 4;
-          epi(mb + m, nb + n, *reinterpret_cast<const float4v*>(rows + m * RP + n));
+          epi(mw + 16 * i + m, nw + n, *reinterpret_cast<const float4v*>(rows + m * RP + n));
         }
-      } else {
-#pragma unroll
-        for (int q0 = 0; q0 < 4 * TW; q0 += 64) {
-          const int q = q0 + lane;
-          if (4 * TW % 64 != 0 && q >= 4 * TW) continue;
-          const int m = q % 4 * 4, n = q / 4;
-          const float* c = rows + m * RP + n;
-          epi_t(mb + m, nb + n, float4v{c[0], c[RP], c[2 * RP], c[3 * RP]});
-        }
+        __builtin_amdgcn_wave_barrier();
       }
-      __builtin_amdgcn_wave_barrier();
+    } else {
+      // columns of the wave's whole tile, in its storage type (what the
+      // epilogue reads of a product): a store covers up to 128 bytes of each,
+      // 32 with 16 rows at a time (merged q/k/v of 16384 rows 87 us so, 75 now)
+      constexpr int TR = COLS ? TM / WM : 16, CP = TR + 4;
+      T* cols = reinterpret_cast<T*>(lds) + w * TW * CP;
+#pragma unroll
+      for (int i0 = 0; i0 < RA; i0 += TR / 16) {
+#pragma unroll
+        for (int i = 0; i < TR / 16; ++i)
+#pragma unroll
+          for (int j = 0; j < RB; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              st(cols + (16 * j + 4 * g + e) * CP + 16 * i + r, acc[i0 + i][j][e]);
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q0 = 0; q0 < TW * TR / 4; q0 += 64) {
+          const int q = q0 + lane;
+          if (TW * TR / 4 % 64 != 0 && q >= TW * TR / 4) continue;
+          const int m = q % (TR / 4) * 4, n = q / (TR / 4);
+          float c[4];
+          load_pack<4>(c, cols + n * CP + m);
+          epi_t(mw + 16 * i0 + m, nw + n, float4v{c[0], c[1], c[2], c[3]});
+        }
+        __builtin_amdgcn_wave_barrier();
+      }
     }
   } else {
     constexpr int P = TN + 4;
