@@ -26,7 +26,8 @@ The MI355X design:
   workgroup; wider rows span whole waves and combine through LDS.
 * **streamed reduction** (rows longer than ``max_persistent_row``): one row
   per 256-thread workgroup, one chunked pass over HBM per reduce (or one
-  online-softmax pass for max+sum(exp)), then a store pass.
+  online-softmax pass for max+sum(exp)), then a store pass; up to 65536
+  elements the row stays in one 1024-lane workgroup's registers instead.
 
 Identical kernel bodies (every transformer layer repeats the same ones) are
 emitted once and shared by name.

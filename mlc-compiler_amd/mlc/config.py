@@ -19,10 +19,13 @@ class Config:
     recompute: bool = True
     reduction_fusion: bool = True
     memory_planning: bool = True
-    #: replay the schedule as one captured hipGraph
+    #: replay the schedule as one captured hipGraph (a short one is launched
+    #: kernel by kernel where that is faster); off: the planned launches, inputs
+    #: copied in
     cuda_graphs: bool = True
     #: fold a bias add that would be a kernel of its own back into the GEMM
-    #: before it (addmm: hipBLASLt's bias epilogue). A schedule change, so it
+    #: before it (addmm), and run the pointwise kernels that directly follow a
+    #: product in its epilogue (``passes/products``). A schedule change, so it
     #: is off by default, where the schedule is the reference's.
     gemm_epilogue: bool = False
     #: merge a pointwise producer into the copy that re-lays its output out

@@ -6,7 +6,8 @@ When nothing fuses with it -- BERT's q/k/v projections, where the add ends up
 as a kernel of its own -- that split costs a launch and a round trip of the
 GEMM output through HBM. This pass puts such an add back into the library
 call: ``mm`` followed by a lone ``out = mm_out + bias`` kernel becomes one
-``addmm(bias, a, b)`` extern (hipBLASLt applies the bias in its epilogue).
+``addmm(bias, a, b)`` extern (the bias is added in the product's epilogue,
+by the native kernel or by hipBLASLt).
 
 It runs after lowering and before planning, so the arena is planned for the
 new schedule. Rounding differs from the split form (the GEMM result is not
