@@ -424,15 +424,20 @@ class CompiledModel:
             out.append(p)
         return out
 
-    def _call_directly(self, inputs, stream: int) -> None:
+    def _call_directly(self, inputs, stream) -> None:
         ptrs = self._in_place(inputs)
         if ptrs is None:
             for dst, src in zip(self._buffers.inputs, inputs):
                 dst.copy_(src.reshape(-1), non_blocking=True)
             ptrs = [t.data_ptr() for t in self._buffers.inputs]
-        self._module.call(self._runs, ptrs, stream)
+        else:
+            # read until the pass ends: the caller may drop an input of another
+            # stream as soon as the call returns
+            for t in inputs:
+                t.record_stream(stream)
+        self._module.call(self._runs, ptrs, stream.cuda_stream)
 
-    def _replay(self, inputs, stream: int) -> None:
+    def _replay(self, inputs, stream) -> None:
         """The inputs into their buffers, then the graph: plain device tensors
         in one launch with it, others through torch."""
         copies = []
@@ -443,7 +448,7 @@ class CompiledModel:
                 copies.append((own.data_ptr(), t.data_ptr(), own.numel() * own.element_size()))
             else:
                 own.copy_(t.reshape(-1), non_blocking=True)
-        self._module.graph_call(copies, stream)
+        self._module.graph_call(copies, stream.cuda_stream)
 
     def run_one(self, k, table: dict[str, torch.Tensor]) -> None:
         if isinstance(k, ExternKernel):
@@ -499,19 +504,20 @@ class CompiledModel:
             self._check_inputs(inputs)
             if self._plan is None:
                 self._resolve(self._buffers.resident(inputs))
-            stream = torch.cuda.current_stream(self.device).cuda_stream
             if self._direct:
                 if self._static_outputs is None:
                     self._static_outputs = self._collect(self._buffers.table)
-                if torch.cuda.current_device() == self._module.index:
-                    self._call_directly(inputs, stream)
-                else:
-                    with torch.cuda.device(self.device):
-                        self._call_directly(inputs, stream)
+                run = self._call_directly
             else:
                 if not self._captured:
                     self._capture(inputs)
-                self._replay(inputs, stream)
+                run = self._replay
+            stream = torch.cuda.current_stream(self.device)
+            if torch.cuda.current_device() == self._module.index:
+                run(inputs, stream)
+            else:
+                with torch.cuda.device(self.device):
+                    run(inputs, stream)
             out = self._static_outputs
         if self.cfg.sync_input_checks:
             self.check_errors()

@@ -92,6 +92,24 @@ def test_another_stream_and_device_order():
     assert _same(got, want)
 
 
+def test_an_input_of_another_stream_may_be_dropped():
+    x, y = _args()
+    compiled = mlc.compile(Chain(), (x, y))
+    want = [t.clone() for t in compiled(x, y)]
+    z = x.clone()
+    at = z.data_ptr()
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(2_000_000)  # the pass is still to come when z goes
+        got = compiled(z, y)
+    del z
+    fresh = torch.full_like(x, 7.0)
+    assert fresh.data_ptr() != at
+    side.synchronize()
+    assert _same(got, want)
+
+
 def test_when_a_graph_is_kept():
     x, _ = _args()
     identity = mlc.compile(Identity(), (x,))
