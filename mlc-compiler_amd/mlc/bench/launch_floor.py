@@ -15,7 +15,7 @@ on the replay stream):
   and workgroup size (the cost of dispatching its waves);
 * ``library calls + empty``: the forward with every generated kernel (and the
   native embedding gather) replaced by a one-workgroup empty node, the
-  library GEMMs real -- what the forward would cost if the fused kernels
+  GEMMs, library or native, real -- what the forward would cost if the fused kernels
   were free;
 * ``library calls only``: the GEMMs alone;
 * ``forward``: every node real (the executor's graph, re-captured here);
@@ -142,9 +142,9 @@ def decompose_compiled(compiled, inputs, replays: int = 200, families=None, shap
     for k, (kind, payload) in zip(compiled.schedule.kernels, compiled._plan):
         if kind == "kernel":
             entries.append(("gen", payload, rt.launch_table[k.name].symbol))
-        elif kind == "extern" and getattr(payload, "module", None) is rt:
+        elif kind == "extern" and k.name in rt.launch_table and getattr(payload, "module", None) is rt:
             entries.append(("gen", payload.bound, rt.launch_table[k.name].symbol))
-        elif kind == "extern":
+        elif kind == "extern":  # a product, by the library or by a native kernel
             entries.append(("lib", payload, None))
     n_gen = sum(1 for e in entries if e[0] == "gen")
     n_lib = len(entries) - n_gen

@@ -158,3 +158,16 @@ def test_batched_in_every_order(shape, orders, dtype):
         args.append(torch.randn(*stored).to(dtype).cuda())
     a, b = (t.double().cpu().permute(o) for t, o in zip(args, orders))
     _check(Batched(*orders), tuple(args), a @ b, a.abs() @ b.abs(), K)
+
+
+@pytest.mark.gpu
+def test_launch_floor_counts_native_products():
+    """The graph decomposition takes a native product as a product, in every graph."""
+    from mlc.bench.launch_floor import decompose_compiled
+
+    torch.manual_seed(0)
+    lin = torch.nn.Linear(128, 128).half().cuda()
+    x = torch.randn(128, 128, device="cuda", dtype=torch.float16)
+    compiled = mlc.compile(torch.nn.Sequential(lin, torch.nn.ReLU()), (x,))
+    d = decompose_compiled(compiled, (x,), replays=2, shapes=False, log=lambda line: None)
+    assert compiled._module.product_table and d["library"] >= 1 and d["generated"] >= 1
