@@ -424,9 +424,13 @@ def _part_lines(part, i: int, N: int, TN: int, along_m: bool = False) -> list[st
     terms = (*part.m_terms, *part.n_terms)
     packed = along_m or (inner[2] == 1 and inner[0] % 4 == 0
                          and all(t is inner or t[2] % 4 == 0 for t in terms))
-    L += [f"        o[j] = {code};", "      }",
-          f"      {STORAGE[out.dtype]}* w = o{i} + (({_place(part.m_terms, 'row')}) "
-          f"+ ({_place(part.n_terms, 'q')}));"]
+    L += [f"        o[j] = {code};", "      }"]
+    if not along_m and inner[0] % 4:  # the four columns may run on into the next digit
+        return L + ["#pragma unroll", "      for (int j = 0; j < 4; ++j)",
+                    f"        mlc::st(o{i} + (({_place(part.m_terms, 'row')}) "
+                    f"+ ({_place(part.n_terms, '(q + j)')})), o[j]);", "    }"]
+    L.append(f"      {STORAGE[out.dtype]}* w = o{i} + (({_place(part.m_terms, 'row')}) "
+             f"+ ({_place(part.n_terms, 'q')}));")
     if packed:
         L.append("      mlc::store_pack<4>(w, o);")
     else:

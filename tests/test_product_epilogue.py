@@ -2,6 +2,8 @@
 (``Config.gemm_epilogue``): which groups form, that a tile's coordinates give
 every operand the element its own index map names, and the results."""
 
+import re
+
 import pytest
 import torch
 import torch.nn as nn
@@ -9,6 +11,7 @@ import torch.nn.functional as F
 
 import mlc
 from mlc.api import build_pipeline
+from mlc.codegen.hip_gemm import emit_group
 from mlc.config import Config
 from mlc.ir.capture import capture
 from mlc.kernels import ExternKernel
@@ -75,6 +78,23 @@ class TwiceRead(nn.Module):
         return torch.relu(y) * 2.0, y.sum(-1)
 
 
+class HeadSize(nn.Module):
+    """A product re-laid out per head; ``act``: with a bias and ReLU on the way."""
+
+    def __init__(self, heads, size, act):
+        super().__init__()
+        self.heads, self.size, self.act = heads, size, act
+        self.lin = nn.Linear(64, heads * size, bias=act)
+
+    def forward(self, x):
+        y = self.lin(x)
+        y = torch.relu(y) if self.act else y
+        return y.view(*x.shape[:2], self.heads, self.size).transpose(1, 2).contiguous()
+
+
+HEAD_SIZES = [(2, 6), (4, 2), (2, 10), (4, 7), (2, 8), (4, 16)]
+
+
 def cases(dtype=torch.float16):
     def r(*s):
         return torch.randn(*s).to(dtype)
@@ -114,6 +134,44 @@ def test_groups_and_their_addresses(at):
                             read.base + read.row * m + read.col * (n - part.lo), name
 
 
+def _stored_at(text, part, i, m, n, along_m):
+    """Where the emitted source stores the four elements it holds at (m, n):
+    columns n to n + 3 of row m (rows m to m + 3 of column n)."""
+    def at(expr, **names):
+        return eval(re.sub(r"(\d)u\b", r"\1", expr).replace("/", "//"), {}, names)
+
+    q = n - part.lo
+    body = text.split("auto store_t =")[1] if along_m else text.split("auto store_t =")[0]
+    start = re.search(rf"\* w = o{i} \+ (.*);\n", body)
+    store = body[start.end() if start else 0:]
+    if start and "store_pack<4>(w, o)" in store.split("    }\n")[0]:
+        first = at(start[1], row=m, q=q)
+        assert first % 4 == 0  # a pack is one aligned access
+        return [first + j for j in range(4)]
+    if start:
+        step = int(re.search(r"st\(w \+ j \* (\d+), o\[j\]\)", store)[1])
+        return [at(start[1], row=m, q=q) + j * step for j in range(4)]
+    each = re.search(rf"mlc::st\(o{i} \+ (.*), o\[j\]\);", body)[1]
+    return [at(each, row=m, q=q, j=j) for j in range(4)]
+
+
+@pytest.mark.parametrize("act", [False, True])
+@pytest.mark.parametrize("heads,size", HEAD_SIZES)
+def test_every_element_is_stored_at_its_own_place(heads, size, act):
+    """The four-wide store as emitted, for heads that a group of four columns
+    ends inside of: each element of the output written once, by its owner."""
+    sched = _schedule(HeadSize(heads, size, act), (torch.zeros(2, 8, 64, dtype=torch.float16),))
+    (i, (_, parts)), = sched.merged.items()
+    y, (part,) = sched.kernels[i].outputs[0], parts
+    text, _ = emit_group(sched.kernels[i], parts)
+    own = next(a for a, read in zip(part.kernel.inputs, part.reads) if read is None)
+    place = {own.index.evaluate(idx=idx): idx for idx in range(part.kernel.numel)}
+    for m in range(y.shape[0]):
+        for n in range(part.lo, part.hi, 4):
+            assert _stored_at(text, part, 0, m, n, False) == \
+                [place[m * y.shape[1] + n + j] for j in range(4)], (m, n)
+
+
 def test_a_group_keeps_its_buffers_alive_throughout():
     """The down projection's residual and input outlive the group's output's
     first write: no two of them share arena bytes."""
@@ -145,6 +203,20 @@ def test_results(at, dtype):
     ulp = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
     err = (got.double().cpu() - want).abs().max() / want.abs().max()
     assert err <= 4 * ulp, (name, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("heads,size", HEAD_SIZES)
+def test_results_by_head_size(heads, size):
+    """Against float64: two roundings to fp16 (product, then bias and ReLU)
+    over sums of 64 products; a misplaced element is off by its own size."""
+    torch.manual_seed(0)
+    model, x = HeadSize(heads, size, True).half(), torch.randn(2, 33, 64).half()
+    want = model.double()(x.double())
+    x, model = x.cuda(), model.half().cuda()
+    compiled = mlc.compile(model, (x,), ALL)
+    assert compiled.schedule.merged
+    assert (compiled(x).double().cpu() - want).abs().max() <= 2.0 ** -9 * want.abs().max()
 
 
 @pytest.mark.gpu
