@@ -93,11 +93,13 @@ __device__ __forceinline__ void gemm_tile(const T* __restrict__ a, const T* __re
   constexpr int STAGE = ROWS * PIECE;
   constexpr int PART = WK > 1 ? WK * TM * (TN + 4) * 4 : 0;
   constexpr int TW = TN / WN, RP = TW + 4, ROWBUF = 16 * RP;   // floats of a wave's row buffer
-  constexpr int EPI = WK > 1 ? PART : GW * ROWBUF * 4;
+  // the column buffer of 16 rows is the larger one in fp32, and more than the
+  // ring where k is one stage of a 256 x 256 tile
+  constexpr int ROWBUFS = GW * ROWBUF * 4, COLBUFS = GW * TW * 20 * (int)sizeof(T);
+  constexpr int EPI = WK > 1 ? PART : ROWBUFS > COLBUFS ? ROWBUFS : COLBUFS;
   constexpr int LDS = WK * RING * STAGE > EPI ? WK * RING * STAGE : EPI;
   // whether the columns of every wave's tile fit at once (16 rows always do)
   constexpr bool COLS = GW * TW * (TM / WM + 4) * (int)sizeof(T) <= LDS;
-  static_assert(GW * TW * 20 * (int)sizeof(T) <= LDS || WK > 1, "column buffer");
   __shared__ __attribute__((aligned(1024))) char lds[LDS];
 
   const int lane = threadIdx.x & 63;

@@ -6,10 +6,12 @@ import torch
 
 import mlc
 from mlc.api import build_pipeline
-from mlc.codegen.hip_gemm import choose_tile, plan_product
+from mlc.codegen.hip_backend import PRELUDE
+from mlc.codegen.hip_gemm import MERGED_FLOPS, TILED_FLOPS, choose_tile, emit_product, plan_product
 from mlc.config import Config
 from mlc.ir.capture import capture
 from mlc.kernels import ExternKernel
+from mlc.runtime import native
 from mlc.runtime.executor import ProductCall
 
 CFG = Config(cuda_graphs=False, gemm_epilogue=True)
@@ -72,10 +74,12 @@ def test_which_calls_run_natively():
 def test_every_tile_splits_its_product(size):
     """The tile chosen for any size divides among its waves and its k-splits
     and fits LDS (the template's own static conditions)."""
-    for M in (1, 2, 15, 16, 17, 33, 64, 100, 128, 197, 300, 512, 1182, 2048):
-        for N in (1, 16, 48, 64, 197, 768, 2304, 3072):
+    for M in (1, 2, 15, 16, 17, 33, 64, 100, 128, 197, 300, 512, 1182, 2048, 4096, 20480):
+        for N in (1, 16, 48, 64, 197, 512, 768, 2304, 3072, 4096):
             for K in (128 // size * n for n in (1, 2, 3, 5, 7, 8, 12, 48)):
-                for batches in (1, 12):
+                for batches in (1, 12, 64, 256):
+                    if 2.0 * batches * M * N * K > max(TILED_FLOPS[size], MERGED_FLOPS):
+                        continue
                     tile, pieces = choose_tile(M, N, K, batches, size), K * size // 128
                     if tile is None:  # few fp32 rows need a k-split of 4
                         assert size == 4 and M <= 128 and pieces % 4
@@ -85,7 +89,39 @@ def test_every_tile_splits_its_product(size):
                     assert TM % (16 * WM) == 0 and TN % (16 * WN) == 0 and WM * WN * WK <= 16
                     ring = min(stages, pieces // WK) * WK * (TM + TN) * 128
                     assert 2 <= stages <= 4 and ring <= 160 * 1024
-                    assert WK == 1 or WK * TM * (TN + 4) * 4 <= 160 * 1024
+                    epilogue = WK * TM * (TN + 4) * 4 if WK > 1 else \
+                        max(WM * 16 * (TN + 4 * WN) * 4, WM * TN * 20 * size)
+                    assert epilogue <= 160 * 1024
+
+
+def _largest(size):
+    """Products up to the operations line, by tile, that take a tile of 64 x 64
+    or more over one piece of k: the ring is at its smallest."""
+    K, found = 128 // size, {}
+    for M in (33, 100, 300, 512, 2048, 4096, 20480):
+        for N in (48, 197, 512, 768, 3072, 4096):
+            for batches in (1, 64):
+                tile = choose_tile(M, N, K, batches, size)
+                if 2.0 * batches * M * N * K <= TILED_FLOPS[size] and tile[0] * tile[1] >= 64 * 64:
+                    found.setdefault(tile, (batches, M, N, K))
+    return found
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+def test_the_large_tiles_compile_over_one_piece_of_k(dtype):
+    """The template's conditions on the tile that is chosen, by the compiler:
+    with one stage the epilogue's buffers are more of LDS than the ring is."""
+    bodies = []
+    found = _largest(dtype.itemsize)
+    assert any(t[:2] == (256, 256) for t in found)
+    for tile, (B, M, N, K) in found.items():
+        model, args = Batched((0, 1, 2), (0, 2, 1)), (torch.empty(B, M, K, dtype=dtype, device="meta"),
+                                                      torch.empty(B, N, K, dtype=dtype, device="meta"))
+        sched = build_pipeline(capture(model, args), CFG)
+        body, spec = emit_product(next(k for k in sched.kernels if isinstance(k, ExternKernel)))
+        assert spec.meta["form"] == ("tiled", *tile)
+        bodies.append(body.replace("KERNEL(", f"product{len(bodies)}(", 1))
+    native.compile_code_object("\n\n".join([PRELUDE, '#include "mlc_gemm.h"', *bodies]) + "\n")
 
 
 def _check(model, args, want, magnitude, K):
