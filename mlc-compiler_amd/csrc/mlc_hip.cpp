@@ -10,6 +10,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -425,14 +426,20 @@ int mlc_plan_call(mlc_plan* plan, int begin, int end, const void* const* inputs,
   if (begin < 0 || end < begin || static_cast<size_t>(end) > plan->entries.size())
     return fail(MLC_E_RANGE, "mlc_plan_call: range out of bounds");
   // the plan stays as it is: concurrent calls each patch a copy of their own
-  unsigned char args[1024];
+  // (a fused kernel has any number of operands: past 128 the copy is allocated)
+  unsigned char few[1024];
   for (int i = begin; i < end; ++i) {
     const Entry& e = plan->entries[static_cast<size_t>(i)];
     if (e.fn == nullptr) return fail(MLC_E_STATE, "mlc_plan_call: entry was never set");
     const unsigned char* at = e.args.data();
+    std::unique_ptr<unsigned char[]> many;
     if (!e.inputs.empty()) {
-      if (e.args.size() > sizeof(args))
-        return fail(MLC_E_RANGE, "mlc_plan_call: an entry's arguments are too long to patch");
+      unsigned char* args = few;
+      if (e.args.size() > sizeof(few)) {
+        many.reset(new (std::nothrow) unsigned char[e.args.size()]);
+        if (many == nullptr) return fail(MLC_E_STATE, "mlc_plan_call: out of host memory");
+        args = many.get();
+      }
       std::memcpy(args, e.args.data(), e.args.size());
       for (const auto& p : e.inputs) {
         if (p.second >= n_inputs) return fail(MLC_E_RANGE, "mlc_plan_call: too few inputs");

@@ -60,6 +60,22 @@ def test_every_kind_of_input():
         assert _same(compiled(x, y), want), name
 
 
+def test_a_kernel_of_many_operands():
+    """One launch of more than 128 pointers (1 KiB of arguments)."""
+    class Sum(nn.Module):
+        def forward(self, *xs):
+            return sum(xs[1:], xs[0] * 2.0)
+
+    torch.manual_seed(0)
+    xs = tuple(torch.randn(8, 64, device="cuda") for _ in range(150))
+    compiled = mlc.compile(Sum(), xs)
+    want = mlc.compile(Sum(), xs, Config(cuda_graphs=False))(*xs).clone()
+    assert torch.equal(compiled(*xs), want) and compiled._direct
+    odd = torch.empty(8 * 64 + 1, device="cuda")
+    odd[1:] = xs[7].reshape(-1)
+    assert torch.equal(compiled(*xs[:7], odd[1:].view(8, 64), *xs[8:]), want)
+
+
 def test_an_output_fed_back_is_copied_first():
     x, y = _args()
     compiled = mlc.compile(Chain(), (x, y))
