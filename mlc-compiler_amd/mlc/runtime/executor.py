@@ -300,6 +300,8 @@ class CompiledModel:
         self._direct = False
         #: memory of this model that a caller's input may be a view of
         self._own: list[tuple[int, int]] = []
+        #: input buffers that outputs are views of (``_shown_inputs``)
+        self._shown: list[tuple[int, int]] | None = None
         self._captured = False
         self._capture_stream = None
         self._static_outputs: Any = None
@@ -439,7 +441,14 @@ class CompiledModel:
 
     def _replay(self, inputs, stream) -> None:
         """The inputs into their buffers, then the graph: plain device tensors
-        in one launch with it, others through torch."""
+        in one launch with it, others through torch. Those copies have no order
+        among them, so an output that is a view of an input's buffer (a model
+        that returns its input) is set aside before it is fed back."""
+        shown = self._shown_inputs()
+        if shown:
+            inputs = [t.clone() if t.device == own.device
+                      and any(lo <= t.data_ptr() < hi for lo, hi in shown) else t
+                      for t, own in zip(inputs, self._buffers.inputs)]
         copies = []
         for t, own in zip(inputs, self._buffers.inputs):
             if (type(t) is torch.Tensor and t.dtype == own.dtype and t.device == own.device
@@ -449,6 +458,15 @@ class CompiledModel:
             else:
                 own.copy_(t.reshape(-1), non_blocking=True)
         self._module.graph_call(copies, stream.cuda_stream)
+
+    def _shown_inputs(self) -> list[tuple[int, int]]:
+        """Address ranges of the inputs' buffers that outputs are views of."""
+        if self._shown is None:
+            outputs = {v.buffer.name for v in self.graph.outputs}
+            self._shown = [(t.data_ptr(), t.data_ptr() + t.numel() * t.element_size())
+                           for v, t in zip(self.graph.inputs, self._buffers.inputs)
+                           if v.buffer.name in outputs]
+        return self._shown
 
     def run_one(self, k, table: dict[str, torch.Tensor]) -> None:
         if isinstance(k, ExternKernel):

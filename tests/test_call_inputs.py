@@ -1,0 +1,67 @@
+"""What a call does with the caller's inputs before its kernels run, on the
+CPU: the executor's own code with a stand-in for the native launches."""
+
+import ctypes
+from types import SimpleNamespace
+
+import pytest
+import torch
+import torch.nn as nn
+
+from mlc.api import build_pipeline
+from mlc.config import Config
+from mlc.ir.capture import capture
+from mlc.runtime.executor import CompiledModel
+from oracle import TorchReferenceRunner
+
+CFG = Config(cuda_graphs=False)
+STREAM = SimpleNamespace(cuda_stream=0)
+
+
+class _Replaying(TorchReferenceRunner):
+    """The copies of ``graph_call`` have no order among them: run here in the
+    given one or the other way round."""
+
+    MAX_COPIES = 8
+
+    def __init__(self, backwards=False):
+        self.backwards, self.copies = backwards, []
+
+    def graph_call(self, copies, stream):
+        self.copies = copies
+        for dst, src, nbytes in copies[::-1] if self.backwards else copies:
+            assert dst and src
+            ctypes.memmove(dst, src, nbytes)
+
+
+def _compile(model, args, runner):
+    graph = capture(model, args)
+    compiled = CompiledModel(graph, build_pipeline(graph, CFG), CFG, torch.device("cpu"),
+                             runner=runner)
+    compiled(*args)  # the buffers exist
+    return compiled
+
+
+class Shift(nn.Module):
+    """Hands its second input back."""
+
+    def forward(self, a, b):
+        return b, a + b
+
+
+@pytest.mark.parametrize("strided", [False, True])
+@pytest.mark.parametrize("backwards", [False, True])
+@pytest.mark.parametrize("at", [0, 1])
+def test_a_returned_input_fed_to_another_place(at, backwards, strided):
+    """An output that is a view of an input's own buffer is read before any
+    input is written, whichever copy runs first."""
+    torch.manual_seed(0)
+    a, b, c = (torch.randn(6, 8) for _ in range(3))
+    compiled = _compile(Shift(), (a, b), _Replaying(backwards))
+    shown = compiled(a, b)[0]
+    assert torch.equal(shown, b)
+    fresh = torch.stack([c, c], -1)[..., 0] if strided else c
+    compiled._replay((shown, fresh) if at == 0 else (fresh, shown), STREAM)
+    got = [t.view(6, 8) for t in compiled._buffers.inputs]
+    want = [b, c] if at == 0 else [c, b]
+    assert all(torch.equal(g, w) for g, w in zip(got, want))
