@@ -270,6 +270,15 @@ class _Buffers:
 # the model
 # --------------------------------------------------------------------------
 
+def _plain(t: torch.Tensor, own: torch.Tensor) -> bool:
+    """Whether a kernel may read the caller's ``t`` at its address in the place
+    of the input buffer ``own``: the same bytes, on 16 of them, and in memory
+    at all (torch's efficient zero tensors are not)."""
+    return (type(t) is torch.Tensor and t.dtype == own.dtype and t.device == own.device
+            and t.is_contiguous() and not t.is_neg() and not t._is_zerotensor()
+            and t.data_ptr() % 16 == 0)
+
+
 def _alloc_count(device) -> int:
     return int(torch.cuda.memory_stats(device).get("allocation.all.allocated", 0))
 
@@ -416,12 +425,11 @@ class CompiledModel:
         (an output fed back)."""
         out = []
         for t, own in zip(inputs, self._buffers.inputs):
-            if type(t) is not torch.Tensor or t.dtype != own.dtype or t.device != own.device \
-                    or not t.is_contiguous() or t.is_neg():
+            if not _plain(t, own):
                 return None
             p = t.data_ptr()
             end = p + own.numel() * own.element_size()
-            if p % 16 or any(p < hi and lo < end for lo, hi in self._own):
+            if any(p < hi and lo < end for lo, hi in self._own):
                 return None
             out.append(p)
         return out
@@ -451,9 +459,7 @@ class CompiledModel:
                       for t, own in zip(inputs, self._buffers.inputs)]
         copies = []
         for t, own in zip(inputs, self._buffers.inputs):
-            if (type(t) is torch.Tensor and t.dtype == own.dtype and t.device == own.device
-                    and t.is_contiguous() and not t.is_neg() and t.data_ptr() % 16 == 0
-                    and len(copies) < self._module.MAX_COPIES):
+            if len(copies) < self._module.MAX_COPIES and _plain(t, own):
                 copies.append((own.data_ptr(), t.data_ptr(), own.numel() * own.element_size()))
             else:
                 own.copy_(t.reshape(-1), non_blocking=True)

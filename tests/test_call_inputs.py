@@ -65,3 +65,22 @@ def test_a_returned_input_fed_to_another_place(at, backwards, strided):
     got = [t.view(6, 8) for t in compiled._buffers.inputs]
     want = [b, c] if at == 0 else [c, b]
     assert all(torch.equal(g, w) for g, w in zip(got, want))
+
+
+class Add(nn.Module):
+    def forward(self, a, b):
+        return a + b
+
+
+def test_a_zero_tensor_has_no_memory_to_read():
+    """torch's efficient zero tensors have a null address: they go through
+    torch's own copy, on both ways in."""
+    a = torch.randn(6, 8)
+    compiled = _compile(Add(), (a, a), _Replaying())
+    compiled._buffers.inputs[1].fill_(7.0)
+    zero = torch._efficientzerotensor(6, 8)
+    assert zero.data_ptr() == 0
+    compiled._replay((a, zero), STREAM)
+    assert torch.equal(compiled._buffers.inputs[1], torch.zeros(48))
+    assert compiled._in_place((a, a)) == [a.data_ptr()] * 2
+    assert compiled._in_place((a, zero)) is None
