@@ -53,7 +53,7 @@ def build_pipeline(graph, cfg: Config) -> Schedule:
         fold_bias_epilogues(schedule)
     if cfg.fused_attention:
         fuse_attention(schedule)
-    if cfg.gemm_epilogue:
+    if cfg.gemm_epilogue and cfg.memory_planning:  # unplanned kernels run one by one
         merge_products(schedule)
     plan_memory(graph, schedule, cfg)
     return schedule

@@ -28,6 +28,7 @@ from ..config import Config
 from ..ir.graph import Graph
 from ..ir.types import Buffer
 from ..kernels import Schedule
+from ..runtime.native import STATIC_SLAB_BYTES
 
 #: byte alignment of every arena offset (16-byte packs, library GEMM operands)
 ALIGNMENT = 256
@@ -86,7 +87,8 @@ class AllocationPlan:
 
 def compute_live_ranges(graph: Graph, schedule: Schedule) -> list[LiveRange]:
     """Lifetimes of the plannable buffers, per *buffer* (a view keeps its
-    whole buffer alive), in order of first appearance in the schedule."""
+    whole buffer alive), in order of first appearance in the schedule. The
+    product of a group that runs as one launch is never stored: it has none."""
     first: dict[str, int] = {}
     last: dict[str, int] = {}
     by_name: dict[str, Buffer] = {}
@@ -109,8 +111,10 @@ def compute_live_ranges(graph: Graph, schedule: Schedule) -> list[LiveRange]:
         by_name.setdefault(v.buffer.name, v.buffer)
         last[v.buffer.name] = len(schedule.kernels)
 
+    unstored = {schedule.kernels[i].outputs[0].buffer.name for i in schedule.merged}
     return [LiveRange(buf, first[name], last[name], _round_up(buf.nbytes))
-            for name, buf in by_name.items() if buf.plannable and name in first]
+            for name, buf in by_name.items()
+            if buf.plannable and name in first and name not in unstored]
 
 
 def peak_live_bytes(ranges: list[LiveRange], n_kernels: int) -> int:
@@ -192,6 +196,11 @@ def plan_memory(graph: Graph, schedule: Schedule, cfg: Config) -> AllocationPlan
                 plan.free_at.setdefault(r.end, []).append(r.buffer.name)
     else:
         plan.offsets, plan.arena_bytes = pack(ranges)
+        if schedule.merged and cfg.static_arena and plan.arena_bytes > STATIC_SLAB_BYTES:
+            # a group's outputs beside its inputs may be more than its product
+            # beside either: its kernels one by one may still fit
+            schedule.merged = {}
+            return plan_memory(graph, schedule, cfg)
         clashes = verify(ranges, plan.offsets)
         if clashes:
             raise AssertionError("arena placement overlaps live buffers:\n" + "\n".join(clashes))

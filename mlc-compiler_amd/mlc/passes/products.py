@@ -8,8 +8,10 @@ map that a tile of the result can invert, the runtime runs the group as one
 launch (``codegen/hip_gemm``): the result is rounded to its storage type in
 registers, as the library stores it, and each kernel's body is evaluated on it
 there. The schedule keeps its kernels (per-kernel profiling times them one by
-one); ``Schedule.merged`` names the groups, and the planner keeps every buffer
-of a group alive through all of it.
+one); ``Schedule.merged`` names the groups. The planner keeps every buffer of a
+group alive through all of it and leaves the product out, which is never
+stored: a GPT-2 block's arena is two thirds of what its kernels one by one need
+(b32 s512 fp16: 151 MB for 226).
 """
 
 from __future__ import annotations

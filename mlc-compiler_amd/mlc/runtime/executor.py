@@ -204,6 +204,9 @@ class _Buffers:
             self.live.update(v.buffer.name for v in (*k.reads(), *k.writes()))
         self.params = {v.buffer.name: graph.param_tensors[v.name].to(model.device).contiguous()
                        .reshape(-1) for v in graph.params}
+        #: products of groups that run as one launch, which never stores them
+        self.unstored = {schedule.kernels[i].outputs[0].buffer.name: schedule.kernels[i].outputs[0].buffer
+                         for i in schedule.merged}
         self.arena: torch.Tensor | None = None
         self.table: dict[str, torch.Tensor] | None = None
         self.inputs: list[torch.Tensor] = []
@@ -254,8 +257,22 @@ class _Buffers:
         for b in self.model.graph.buffers():
             if b.name in table or b.name not in self.live:
                 continue
+            if b.name in self.unstored:
+                continue
             at = offsets.get(b.name)
             table[b.name] = self.empty(b) if at is None else arena[at:at + b.nbytes].view(b.dtype)
+
+    def place_unstored(self) -> None:
+        """Memory for the products that only a group's kernels run one by one
+        write and read: one piece for all of them, each is done with by the
+        end of its group."""
+        names = self.unstored.keys() - self.table.keys()
+        if names:
+            piece = torch.empty(max(self.unstored[n].nbytes for n in names), dtype=torch.uint8,
+                                device=self.model.device)
+            for n in names:
+                b = self.unstored[n]
+                self.table[n] = piece[:b.nbytes].view(b.dtype)
 
     def get_arena(self) -> torch.Tensor:
         need = max(self.model.schedule.arena_bytes, 1)
@@ -303,7 +320,8 @@ class CompiledModel:
         self._constants = {k.name for k in schedule.kernels
                            if isinstance(k, ExternKernel) and not k.reads()}
         self._buffers = _Buffers(self)
-        self._plan: list | None = None
+        #: every kernel bound, None where only its group is (``_plan``)
+        self._bindings: list | None = None
         self._runs: list | None = None
         #: inputs are read in place and the runs launched one by one
         self._direct = False
@@ -345,37 +363,56 @@ class CompiledModel:
         return outs[0] if len(outs) == 1 else tuple(outs)
 
     # -- the plan ---------------------------------------------------------------
+    def _bind(self, k, table: dict[str, torch.Tensor]) -> tuple:
+        """``(kind, payload)`` of one kernel, with kind "const" (run once, when
+        the plan is resolved), "extern" or "kernel"."""
+        if isinstance(k, ExternKernel):
+            kind = "const" if k.name in self._constants else "extern"
+            return kind, bind_extern(k, table, self._module)
+        return "kernel", self._module.bind(k, table)
+
+    @property
+    def _plan(self) -> list | None:
+        """Every kernel's binding in schedule order, a group's members one by
+        one, for timing kernels by themselves."""
+        if self._bindings is not None and None in self._bindings:
+            self._buffers.place_unstored()
+            table = self._buffers.table
+            self._bindings = [b or self._bind(k, table)
+                              for k, b in zip(self.schedule.kernels, self._bindings)]
+        return self._bindings
+
     def _resolve(self, table: dict[str, torch.Tensor]) -> None:
-        """Bind every kernel once: ``[(kind, payload)]`` in schedule order,
-        with kind "const" (already run), "extern" or "kernel"."""
-        if self._plan is not None:
+        """Bind every launch of a pass once. A group of kernels that is one
+        launch takes the place of its members, which are bound when
+        ``_plan`` is asked for."""
+        if self._runs is not None:
             return
-        plan = []
-        for k in self.schedule.kernels:
-            if k.name in self._constants:
-                call = bind_extern(k, table, self._module)
-                call.run()
-                plan.append(("const", call))
-            elif isinstance(k, ExternKernel):
-                plan.append(("extern", bind_extern(k, table, self._module)))
-            else:
-                plan.append(("kernel", self._module.bind(k, table)))
-        self._plan = plan
-        # what a pass runs: a group of kernels that is one launch takes the
-        # place of its members
         bind_group = getattr(self._module, "bind_group", None)
-        launches, i = [], 0
-        while i < len(plan):
-            if bind_group is not None and i in self.schedule.merged:
-                launches.append(("kernel", bind_group(self.schedule.kernels[i], table)))
-                i = self.schedule.merged[i][0] + 1
-            else:
-                launches.append(plan[i])
-                i += 1
+        merged = self.schedule.merged if bind_group is not None else {}
+        if len(merged) < len(self.schedule.merged):  # their kernels run one by one
+            self._buffers.place_unstored()
+        bindings: list = [None] * len(self.schedule.kernels)
+        launches, of, i = [], [], 0
+        while i < len(bindings):
+            k = self.schedule.kernels[i]
+            if i in merged:
+                end = merged[i][0]
+                launches.append(("kernel", bind_group(k, table)))
+                of.append(self.schedule.kernels[i:end + 1])
+                i = end + 1
+                continue
+            bindings[i] = self._bind(k, table)
+            if k.name in self._constants:
+                bindings[i][1].run()
+            launches.append(bindings[i])
+            of.append([k])
+            i += 1
+        self._bindings = bindings
         group = getattr(self._module, "compile_runs", None)
         self._runs = group(launches) if group is not None else launches
         if (self.cfg.cuda_graphs and self.device.type == "cuda"
-                and hasattr(self._module, "bind_inputs") and self._launch_directly(launches, table)):
+                and hasattr(self._module, "bind_inputs") and self._launch_directly(launches, of)):
             self._module.bind_inputs(self._runs, {t.data_ptr(): i for i, t in
                                                   enumerate(self._buffers.inputs)})
             mine = {id(t) for t in (*self._buffers.inputs, *self.params.values())}
@@ -384,7 +421,7 @@ class CompiledModel:
                          for t in (*held, *([self._arena] if self._arena is not None else []))]
             self._direct = True
 
-    def _launch_directly(self, launches, table) -> bool:
+    def _launch_directly(self, launches, of) -> bool:
         """Whether a pass launches its kernels one by one on the caller's own
         inputs rather than replaying a graph behind a copy of them.
 
@@ -403,8 +440,8 @@ class CompiledModel:
         writes = [v for k in self.schedule.kernels if k.name not in self._constants
                   for v in k.writes()]
         bound = [c for kind, c in launches if kind == "extern" and isinstance(c, ExternCall)]
-        read = [v for k, (_, c) in zip(self.schedule.kernels, self._plan)
-                if any(c is x for x in bound) for v in k.reads()]
+        read = [v for kernels, (_, c) in zip(of, launches) if any(c is x for x in bound)
+                for k in kernels for v in k.reads()]
         if any(v.buffer.name in names for v in (*self.graph.outputs, *writes, *read)):
             return False
         count = sum(kind != "const" for kind, _ in launches)
@@ -483,7 +520,7 @@ class CompiledModel:
     def run_kernels(self, table: dict[str, torch.Tensor]) -> None:
         """One pass of the schedule over ``table`` (through the resolved plan
         when ``table`` is the resident one)."""
-        if self._plan is not None and table is self._buffers.table:
+        if self._runs is not None and table is self._buffers.table:
             for kind, payload in self._runs:
                 if kind == "extern":
                     payload.run()
@@ -526,7 +563,7 @@ class CompiledModel:
             out = self.forward(*inputs)
         else:
             self._check_inputs(inputs)
-            if self._plan is None:
+            if self._runs is None:
                 self._resolve(self._buffers.resident(inputs))
             if self._direct:
                 if self._static_outputs is None:

@@ -15,6 +15,9 @@ from mlc.codegen.hip_gemm import emit_group
 from mlc.config import Config
 from mlc.ir.capture import capture
 from mlc.kernels import ExternKernel
+from mlc.passes.memory_planning import plan_memory
+from mlc.runtime.native import STATIC_SLAB_BYTES
+from oracle import compile_reference
 
 ALL = Config(cuda_graphs=False, merge_parallel_gemms=True, gemm_epilogue=True,
              layout_selection=True, fused_attention=True)
@@ -27,6 +30,27 @@ class Mlp(nn.Module):
 
     def forward(self, x):
         return x + self.down(F.gelu(self.up(x))) * 0.5
+
+
+class Block(Mlp):
+    """The residual is alive beside the product, as in a GPT-2 block."""
+
+    def forward(self, x):
+        h = torch.tanh(x)
+        return h + self.down(F.gelu(self.up(F.layer_norm(h, h.shape[-1:]))))
+
+
+class FanOut(nn.Module):
+    """Two outputs as wide as the product, from an input four times that."""
+
+    def __init__(self):
+        super().__init__()
+        self.up = nn.Linear(1024, 256, bias=False)
+
+    def forward(self, x):
+        y = self.up(torch.tanh(x))
+        a, b = torch.relu(y), torch.sigmoid(y)
+        return torch.cat([a.sum(-1), b.sum(-1)])
 
 
 class Heads(nn.Module):
@@ -105,8 +129,8 @@ def cases(dtype=torch.float16):
             ("transposed", Transposed(), (r(40, 64),), None), ("twice", TwiceRead(), (r(40, 64),), 0)]
 
 
-def _schedule(model, args):
-    return build_pipeline(capture(model.to(args[0].dtype), args), ALL)
+def _schedule(model, args, cfg=ALL):
+    return build_pipeline(capture(model.to(args[0].dtype), args), cfg)
 
 
 @pytest.mark.parametrize("at", range(6))
@@ -132,6 +156,40 @@ def test_groups_and_their_addresses(at):
                     if read is not None:
                         assert a.index.evaluate(idx=idx) == \
                             read.base + read.row * m + read.col * (n - part.lo), name
+
+
+@pytest.mark.parametrize("model,args", [(c[1], c[2]) for c in cases()[:4]]
+                         + [(Block(), (torch.zeros(40, 64, dtype=torch.float16),))])
+def test_a_group_takes_no_more_memory_than_its_kernels(model, args):
+    """One launch never stores the product: it has no place in the arena."""
+    sched = _schedule(model, args)
+    products = [sched.kernels[i].outputs[0].buffer.name for i in sched.merged]
+    assert products and not set(products) & set(sched.plan.offsets)
+    merged = sched.arena_bytes
+    sched.merged = {}
+    assert merged <= plan_memory(sched.graph, sched, ALL).arena_bytes
+    assert not _schedule(model, args, ALL.replace(memory_planning=False)).merged
+
+
+def test_the_static_arena_holds_what_it_held():
+    """64 MiB hold the kernels one by one (60 MiB) and not the group (72)."""
+    cfg = ALL.replace(static_arena=True, reduction_fusion=False)
+    args = (torch.empty(24 * 1024, 1024, dtype=torch.float16, device="meta"),)
+    with torch.device("meta"):
+        model = FanOut()
+    assert _schedule(model, args, cfg.replace(static_arena=False)).arena_bytes > STATIC_SLAB_BYTES
+    sched = _schedule(model, args, cfg)
+    assert not sched.merged and sched.arena_bytes <= STATIC_SLAB_BYTES
+
+
+@pytest.mark.parametrize("at", range(5))
+def test_a_group_whose_kernels_run_one_by_one(at):
+    """A runner without one-launch groups, and the bindings that timing uses."""
+    _, model, args, _ = cases(torch.float32)[at]
+    got, want = (compile_reference(model.float(), args, c)
+                 for c in (ALL, ALL.replace(gemm_epilogue=False)))
+    assert torch.equal(got(*args), want(*args))
+    assert len(got._plan) == len(got.schedule.kernels) and None not in got._plan
 
 
 def _stored_at(text, part, i, m, n, along_m):
