@@ -389,16 +389,18 @@ class CompiledModel:
         if self._runs is not None:
             return
         bind_group = getattr(self._module, "bind_group", None)
-        merged = self.schedule.merged if bind_group is not None else {}
-        if len(merged) < len(self.schedule.merged):  # their kernels run one by one
+        groups = {i: bind_group(self.schedule.kernels[i], table)
+                  for i in self.schedule.merged} if bind_group is not None else {}
+        groups = {i: bound for i, bound in groups.items() if bound is not None}
+        if len(groups) < len(self.schedule.merged):  # the others' kernels run one by one
             self._buffers.place_unstored()
         bindings: list = [None] * len(self.schedule.kernels)
         launches, of, i = [], [], 0
         while i < len(bindings):
             k = self.schedule.kernels[i]
-            if i in merged:
-                end = merged[i][0]
-                launches.append(("kernel", bind_group(k, table)))
+            if i in groups:
+                end = self.schedule.merged[i][0]
+                launches.append(("kernel", groups[i]))
                 of.append(self.schedule.kernels[i:end + 1])
                 i = end + 1
                 continue

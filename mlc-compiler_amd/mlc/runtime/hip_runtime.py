@@ -69,6 +69,10 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+def _on_16_bytes(spec: LaunchSpec | None, buffers: dict[str, torch.Tensor]) -> bool:
+    return spec is not None and all(buffers[n].data_ptr() % 16 == 0 for n in spec.meta["buffers"])
+
+
 class HipRuntime:
     name = "hip"
 
@@ -155,12 +159,16 @@ class HipRuntime:
 
     def bind_product(self, k: ExternKernel, buffers: dict[str, torch.Tensor]) -> Bound | None:
         """A matrix product this module runs in the library's place, resolved
-        like a generated kernel; ``None`` leaves it to the library."""
-        return self._bind_extern(k, self.product_table.get(k.name), buffers)
+        like a generated kernel; ``None`` leaves it to the library, whose
+        operands may lie anywhere (a weight at an odd place in flat storage)."""
+        spec = self.product_table.get(k.name)
+        return self._bind_extern(k, spec, buffers) if _on_16_bytes(spec, buffers) else None
 
-    def bind_group(self, k: ExternKernel, buffers: dict[str, torch.Tensor]) -> Bound:
-        """The group of kernels starting at ``k`` that runs as one launch."""
-        return self._bind_extern(k, self.group_table[k.name], buffers)
+    def bind_group(self, k: ExternKernel, buffers: dict[str, torch.Tensor]) -> Bound | None:
+        """The group of kernels starting at ``k`` that runs as one launch;
+        ``None`` leaves its kernels apart, as ``bind_product`` does."""
+        spec = self.group_table[k.name]
+        return self._bind_extern(k, spec, buffers) if _on_16_bytes(spec, buffers) else None
 
     def _bind_extern(self, k: ExternKernel, spec: LaunchSpec | None,
                      buffers: dict[str, torch.Tensor]) -> Bound | None:

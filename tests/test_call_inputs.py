@@ -9,9 +9,11 @@ import torch
 import torch.nn as nn
 
 from mlc.api import build_pipeline
+from mlc.codegen.hip_backend import build_products
 from mlc.config import Config
 from mlc.ir.capture import capture
 from mlc.runtime.executor import CompiledModel
+from mlc.runtime.hip_runtime import HipRuntime
 from oracle import TorchReferenceRunner
 
 CFG = Config(cuda_graphs=False)
@@ -65,6 +67,49 @@ def test_a_returned_input_fed_to_another_place(at, backwards, strided):
     got = [t.view(6, 8) for t in compiled._buffers.inputs]
     want = [b, c] if at == 0 else [c, b]
     assert all(torch.equal(g, w) for g, w in zip(got, want))
+
+
+class _Apart(TorchReferenceRunner):
+    """A runtime that cannot run any group as one launch."""
+
+    def bind_group(self, k, buffers):
+        return None
+
+
+def _linear():
+    model = nn.Sequential(nn.Linear(64, 64), nn.ReLU())
+    args = (torch.randn(32, 64),)
+    graph = capture(model, args)
+    return model, args, graph, build_pipeline(graph, CFG.replace(gemm_epilogue=True))
+
+
+def test_a_group_that_cannot_be_bound_runs_its_kernels():
+    model, args, graph, sched = _linear()
+    assert sched.merged
+    compiled = CompiledModel(graph, sched, CFG, torch.device("cpu"), runner=_Apart())
+    torch.testing.assert_close(compiled(*args), model(*args))
+
+
+def test_a_product_off_16_bytes_is_the_librarys():
+    """A weight at an odd place in flat storage, an input view in the unplanned
+    mode: the native kernels' loads need 16-byte aligned buffers, the library's
+    do not."""
+    _, _, _, sched = _linear()
+    module, groups = build_products(sched)
+    at = {v.buffer.name: 4096 * (i + 1) for i, v in enumerate(
+        {v.buffer.name: v for k in sched.kernels for v in (*k.reads(), *k.writes())}.values())}
+    buffers = {v.buffer.name: SimpleNamespace(
+        device=torch.device("cuda"), dtype=v.buffer.dtype, numel=lambda n=v.buffer.numel: n,
+        data_ptr=lambda n=v.buffer.name: at[n])
+        for k in sched.kernels for v in (*k.reads(), *k.writes())}
+    rt = object.__new__(HipRuntime)
+    rt._plans, rt.lib = [], None
+    rt.product_table, rt.group_table = groups, groups  # the same operands either way
+    rt.functions = {spec.symbol: 1 for spec in groups.values()}
+    k = sched.kernels[min(sched.merged)]
+    assert rt.bind_product(k, buffers) is not None and rt.bind_group(k, buffers) is not None
+    at[k.node.args[1].buffer.name] += 2
+    assert rt.bind_product(k, buffers) is None and rt.bind_group(k, buffers) is None
 
 
 class Add(nn.Module):

@@ -196,6 +196,31 @@ def test_batched_in_every_order(shape, orders, dtype):
     _check(Batched(*orders), tuple(args), a @ b, a.abs() @ b.abs(), K)
 
 
+class Stack(torch.nn.Module):
+    def __init__(self, weight):
+        super().__init__()
+        self.weight = torch.nn.Parameter(weight)
+
+    def forward(self, x):
+        return torch.relu(torch.mm(x, self.weight.t())) * 2.0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("cfg", [Config(), CFG, CFG.replace(cuda_graphs=True),
+                                 CFG.replace(memory_planning=False)])
+def test_a_weight_off_16_bytes_goes_to_the_library(cfg):
+    torch.manual_seed(0)
+    flat = torch.randn(96 * 64 + 1, device="cuda", dtype=torch.float16)
+    model = Stack(flat[1:].view(96, 64))
+    x = torch.randn(37, 64, device="cuda", dtype=torch.float16)
+    want = torch.relu(x.double() @ model.weight.double().t()) * 2.0
+    compiled = mlc.compile(model, (x,), cfg)
+    for _ in range(3):
+        got = compiled(x)
+        assert (got.double() - want).abs().max() <= 2.0 ** -10 * want.abs().max()
+        torch.cuda.synchronize()
+
+
 @pytest.mark.gpu
 def test_launch_floor_counts_native_products():
     """The graph decomposition takes a native product as a product, in every graph."""
