@@ -963,6 +963,9 @@ def emit_reduction(k: ReductionKernel, cfg: Config) -> tuple[str, LaunchSpec]:
 #: most this many register elements per lane over the row's column operands
 RESIDENT = {"lanes": 1024, "elements": 64}
 
+#: threads of one launch, which HIP keeps below this
+MAX_THREADS = 2 ** 32
+
 
 def resident_geometry(k: ReductionKernel) -> dict | None:
     """Geometry of a streamed row that fits one workgroup's registers, or
@@ -1002,7 +1005,8 @@ def resident_geometry(k: ReductionKernel) -> dict | None:
     G = RESIDENT["lanes"]
     nvec = -(-C // V) + (1 if shifted else 0)  # a shifted row can touch one pack more
     K = -(-nvec // G)
-    if nvec < 2 * G or K * V * n_loaded > RESIDENT["elements"]:
+    if (nvec < 2 * G or K * V * n_loaded > RESIDENT["elements"]
+            or k.n_rows * G >= MAX_THREADS):
         return None
     return {"G": G, "K": K, "rows_per_wg": 1, "block": G, "V": V,
             "shift": col_args[0] if shifted else None}

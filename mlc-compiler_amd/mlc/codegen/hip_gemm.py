@@ -33,8 +33,8 @@ import torch
 from ..ir.graph import Value
 from ..ir.scalar import Call
 from ..kernels import ExternKernel
-from .hip_backend import (STORAGE, LaunchSpec, Renderer, _subexprs as subexprs, fp16_rounded,
-                          half_inputs, itemsize, value_types_of)
+from .hip_backend import (MAX_THREADS, STORAGE, LaunchSpec, Renderer, _subexprs as subexprs,
+                          fp16_rounded, half_inputs, itemsize, value_types_of)
 
 CUS, XCDS = 256, 8
 LDS_BYTES = 160 * 1024
@@ -235,10 +235,17 @@ def plan_product(k: ExternKernel, merged_flops: float = 0.0, math: bool = False)
             and a.aligned(E, batches) and b.aligned(E, batches)):
         tile = choose_tile(M, N, K, batches, size, math)
         if tile is not None:
-            return Product(batches, M, N, K, a, b, c, bias, ("tiled", *tile))
+            return _launchable(Product(batches, M, N, K, a, b, c, bias, ("tiled", *tile)))
     if rank == 3 and flops <= STAGED_FLOPS:
-        return Product(batches, M, N, K, a, b, c, bias, ("staged", *staged_tile(M, N, batches)))
+        return _launchable(Product(batches, M, N, K, a, b, c, bias,
+                                   ("staged", *staged_tile(M, N, batches))))
     return None
+
+
+def _launchable(p: Product) -> Product | None:
+    """``p`` unless its grid has more threads than HIP launches."""
+    src = _Source(p)
+    return p if src.grid * src.threads < MAX_THREADS else None
 
 
 def staged_tile(M: int, N: int, batches: int) -> tuple[int, int]:

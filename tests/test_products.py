@@ -6,7 +6,7 @@ import torch
 
 import mlc
 from mlc.api import build_pipeline
-from mlc.codegen.hip_backend import PRELUDE
+from mlc.codegen.hip_backend import PRELUDE, emit_kernel
 from mlc.codegen.hip_gemm import MERGED_FLOPS, TILED_FLOPS, choose_tile, emit_product, plan_product
 from mlc.config import Config
 from mlc.ir.capture import capture
@@ -92,6 +92,27 @@ def test_every_tile_splits_its_product(size):
                     epilogue = WK * TM * (TN + 4) * 4 if WK > 1 else \
                         max(WM * 16 * (TN + 4 * WN) * 4, WM * TN * 20 * size)
                     assert epilogue <= 160 * 1024
+
+
+def test_launches_stay_below_two_to_the_32_threads():
+    """HIP's limit for a launch: a batch past it stays with the library, as a
+    reduction over so many resident rows stays with the chunk loop."""
+    def scores(batch):
+        return _form(Batched((0, 1, 2), (0, 1, 2)), torch.empty(batch, 2, 3, dtype=torch.float16, device="meta"),
+                     torch.empty(batch, 3, 2, dtype=torch.float16, device="meta"))
+
+    assert scores((1 << 24) - 8) == "staged" and scores(1 << 24) is None
+
+    class Long(torch.nn.Module):
+        def forward(self, x):
+            return x.sum(-1)
+
+    def resident(rows):
+        x = torch.empty(rows, 40000, dtype=torch.float16, device="meta")
+        k, = build_pipeline(capture(Long(), (x,)), CFG).kernels
+        return emit_kernel(k, CFG)[1].meta["resident"]
+
+    assert resident((1 << 22) - 1) and not resident(1 << 22)
 
 
 def _largest(size):
