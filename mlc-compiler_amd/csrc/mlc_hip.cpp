@@ -10,6 +10,7 @@
 #include <atomic>
 #include <cstdint>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <new>
@@ -372,7 +373,12 @@ int mlc_plan_create(mlc_ctx* ctx, int n_entries, mlc_plan** out) {
   mlc_plan* p = new (std::nothrow) mlc_plan;
   if (p == nullptr) return fail(MLC_E_STATE, "mlc_plan_create: out of host memory");
   p->ctx = ctx;
-  p->entries.resize(static_cast<size_t>(n_entries));
+  try {
+    p->entries.resize(static_cast<size_t>(n_entries));
+  } catch (const std::exception&) {
+    delete p;
+    return fail(MLC_E_STATE, "mlc_plan_create: out of host memory");
+  }
   *out = p;
   return MLC_OK;
 }
@@ -385,12 +391,18 @@ int mlc_plan_set(mlc_plan* plan, int index, mlc_fn fn, uint32_t grid, uint32_t b
   if (grid == 0 || block == 0 || block > 1024)
     return fail(MLC_E_ARG, "mlc_plan_set: bad launch geometry");
   Entry& e = plan->entries[static_cast<size_t>(index)];
+  const unsigned char* b = static_cast<const unsigned char*>(kernarg);
+  try {
+    e.args.assign(b, b + size);
+  } catch (const std::exception&) {
+    e.fn = nullptr;
+    return fail(MLC_E_STATE, "mlc_plan_set: out of host memory");
+  }
+  e.inputs.clear();  // offsets into other arguments
   e.fn = reinterpret_cast<hipFunction_t>(fn);
   e.grid = grid;
   e.block = block;
   e.lds = lds_bytes;
-  const unsigned char* b = static_cast<const unsigned char*>(kernarg);
-  e.args.assign(b, b + size);
   return MLC_OK;
 }
 
@@ -415,7 +427,11 @@ int mlc_plan_input(mlc_plan* plan, int index, uint32_t offset, int input) {
   Entry& e = plan->entries[static_cast<size_t>(index)];
   if (offset % sizeof(void*) != 0 || offset + sizeof(void*) > e.args.size())
     return fail(MLC_E_RANGE, "mlc_plan_input: offset outside the entry's arguments");
-  e.inputs.emplace_back(offset, input);
+  try {
+    e.inputs.emplace_back(offset, input);
+  } catch (const std::exception&) {
+    return fail(MLC_E_STATE, "mlc_plan_input: out of host memory");
+  }
   return MLC_OK;
 }
 

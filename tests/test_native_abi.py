@@ -8,11 +8,13 @@ from __future__ import annotations
 import ctypes
 import re
 import subprocess
+import sys
 
 import pytest
 
 from mlc.runtime import native
 
+MLC_E_STATE = -10003
 HEADER = native.INCLUDE / "mlc_hip.h"
 
 
@@ -68,3 +70,30 @@ def test_check_raises_with_the_library_message(lib):
     rc = lib.mlc_plan_set(None, 0, None, 1, 64, 0, None, 0)
     with pytest.raises(native.NativeError, match="mlc_plan_set"):
         native.check(rc, "mlc_plan_set")
+
+
+def test_no_exception_crosses_the_abi():
+    """Out of host memory is a return code. In a process of its own, whose
+    address space has no room for the entries asked for."""
+    code = f"""
+import ctypes, resource, sys
+sys.path.insert(0, {str(native.ROOT)!r})
+from mlc.runtime import native
+lib = native.load_library()
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (1 << 30), used + (1 << 30)))
+ctx, plan = ctypes.c_void_p(4096), ctypes.c_void_p()  # the context is only kept
+assert lib.mlc_plan_create(ctx, (1 << 31) - 1, ctypes.byref(plan)) == {MLC_E_STATE}
+assert b"out of host memory" in lib.mlc_last_error() and not plan.value
+assert lib.mlc_plan_create(ctx, 1, ctypes.byref(plan)) == 0
+few = ctypes.create_string_buffer(64)
+assert lib.mlc_plan_set(plan, 0, 4096, 1, 64, 0, few, 64) == 0
+assert lib.mlc_plan_set(plan, 0, 4096, 1, 64, 0, few, 1 << 40) == {MLC_E_STATE}
+assert lib.mlc_plan_input(plan, 0, 56, 3) == 0
+assert lib.mlc_plan_input(plan, 0, 60, 3) == -10002
+assert lib.mlc_plan_set(plan, 0, 4096, 1, 64, 0, few, 8) == 0  # forgets the inputs
+assert lib.mlc_plan_input(plan, 0, 8, 0) == -10002
+lib.mlc_plan_destroy(plan)
+"""
+    proc = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr
