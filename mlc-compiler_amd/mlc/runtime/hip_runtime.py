@@ -195,6 +195,10 @@ class HipRuntime:
         """Whether a kernel of this module can flag an invalid input."""
         return self._error_word is not None
 
+    def fetch_errors(self, stream: int | None = None) -> None:
+        """Nothing to enqueue: the word is host memory that kernels write. Kept
+        for callers of the time when a run copied it back."""
+
     def pending_error(self) -> str | None:
         """The message for an invalid input flagged by a completed run, read
         without waiting for the device; ``None`` if no completed run flagged

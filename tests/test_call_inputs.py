@@ -129,3 +129,9 @@ def test_a_zero_tensor_has_no_memory_to_read():
     assert torch.equal(compiled._buffers.inputs[1], torch.zeros(48))
     assert compiled._in_place((a, a)) == [a.data_ptr()] * 2
     assert compiled._in_place((a, zero)) is None
+
+
+def test_the_seams_methods_for_invalid_inputs():
+    for name in ("fetch_errors", "pending_error", "clear_errors", "check_errors"):
+        assert callable(getattr(HipRuntime, name))
+    assert object.__new__(HipRuntime).fetch_errors(0) is None  # nothing to enqueue
