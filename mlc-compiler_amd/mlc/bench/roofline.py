@@ -35,6 +35,21 @@ def distinct_elements(imap: IndexMap) -> int:
     return math.prod(size for a in imap.axes for size, _, _ in a.terms)
 
 
+def _reads(k) -> dict:
+    """Bytes of every distinct operand view of a kernel, by buffer and view."""
+    if isinstance(k, ExternKernel):
+        return {(v.buffer.name, v.layout): v.numel * _itemsize(v.dtype) for v in k.inputs}
+    return {(a.value.buffer.name, a.index.render()): distinct_elements(a.index) * _itemsize(a.dtype)
+            for a in k.inputs}
+
+
+def _writes(k) -> dict:
+    if isinstance(k, ExternKernel):
+        return {(v.buffer.name, v.layout): v.numel * _itemsize(v.dtype) for v in k.outputs}
+    return {(a.value.buffer.name, a.index.render()): distinct_elements(a.index) * _itemsize(a.dtype)
+            for a in k.outputs}
+
+
 def algorithmic_bytes(k) -> int:
     if isinstance(k, ExternKernel):
         if k.node.op == "aten.embedding.default":
@@ -44,43 +59,33 @@ def algorithmic_bytes(k) -> int:
         raise TypeError(f"no byte model for extern {k.node.op}")
     if not isinstance(k, (PointwiseKernel, ReductionKernel, AttentionKernel)):
         raise TypeError(type(k).__name__)
-    seen = set()
-    total = 0
-    for a in k.inputs:
-        key = (a.value.buffer.name, a.index.render())
-        if key in seen:
-            continue
-        seen.add(key)
-        total += distinct_elements(a.index) * _itemsize(a.dtype)
-    for a in k.outputs:
-        total += distinct_elements(a.index) * _itemsize(a.dtype)
-    return total
+    return sum(_reads(k).values()) + sum(_writes(k).values())
 
 
 def extern_bytes(k: ExternKernel) -> int:
     """Algorithmic bytes of a library call: every distinct operand view read
     once (a GEMM's weights included) plus every output written once."""
-    seen = set()
-    total = 0
-    for v in k.inputs:
-        key = (v.buffer.name, v.layout)
-        if key in seen:
-            continue
-        seen.add(key)
-        total += v.numel * _itemsize(v.dtype)
-    for v in k.outputs:
-        total += v.numel * _itemsize(v.dtype)
-    return total
+    return sum(_reads(k).values()) + sum(_writes(k).values())
+
+
+def launch_bytes(kernels) -> int:
+    """Algorithmic bytes of one launch: a kernel's, or those of a product and
+    the pointwise kernels after it as one, which never stores the product and
+    reads what several of them read once."""
+    first = kernels[0]
+    if len(kernels) == 1:
+        gather = isinstance(first, ExternKernel) and first.node.op == "aten.embedding.default"
+        return algorithmic_bytes(first) if gather or not isinstance(first, ExternKernel) \
+            else extern_bytes(first)
+    product = first.outputs[0].buffer.name
+    views: dict = {}
+    for k in kernels:
+        views.update(_reads(k) | _writes(k))
+    return sum(n for (name, _), n in views.items() if name != product)
 
 
 def forward_bytes(schedule) -> int:
     """Algorithmic bytes of one whole forward: every kernel, generated or
     library, at its algorithmic traffic. Divided by the HBM peak it is the
     bytes-moved floor of the forward's latency."""
-    total = 0
-    for k in schedule.kernels:
-        if isinstance(k, ExternKernel) and k.node.op != "aten.embedding.default":
-            total += extern_bytes(k)
-        else:
-            total += algorithmic_bytes(k)
-    return total
+    return sum(launch_bytes([k]) for k in schedule.kernels)

@@ -448,14 +448,18 @@ class CompiledModel:
             return False
         count = sum(kind != "const" for kind, _ in launches)
         host = 3.0 * (count - len(bound)) + 9.0 * len(bound)
-        return count <= MAX_DIRECT and host <= max(24.0, self._device_estimate(count))
+        work = [kernels for kernels, (kind, _) in zip(of, launches) if kind != "const"]
+        return count <= MAX_DIRECT and host <= max(24.0, self._device_estimate(work))
 
-    def _device_estimate(self, count: int) -> float:
-        """Microseconds the device is busy with a pass, at least: the launches'
-        floor, and their buffers at 5 TB/s."""
-        moved = sum(v.buffer.nbytes for k in self.schedule.kernels if k.name not in self._constants
-                    for v in (*k.reads(), *k.writes()))
-        return 1.5 * count + moved / 5e6
+    @staticmethod
+    def _device_estimate(launches) -> float:
+        """Microseconds the device is busy with a pass, by what it cannot do
+        without: the launches' floor, and the bytes that each launch reads and
+        writes (the rows a gather picks, not its table; a group's operands, not
+        its product) at 5 TB/s."""
+        from ..bench.roofline import launch_bytes
+
+        return 1.5 * len(launches) + sum(map(launch_bytes, launches)) / 5e6
 
     def _in_place(self, inputs) -> list[int] | None:
         """Addresses of the caller's inputs, or ``None`` when one of them has to

@@ -5,11 +5,14 @@ survey of the reference derives for each benchmark configuration."""
 from __future__ import annotations
 
 import pytest
+import torch
 
 from mlc.api import build_pipeline
-from mlc.bench.roofline import algorithmic_bytes, extern_bytes, forward_bytes
+from mlc.bench.roofline import algorithmic_bytes, extern_bytes, forward_bytes, launch_bytes
 from mlc.config import Config
+from mlc.ir.capture import capture
 from mlc.kernels import ExternKernel, PointwiseKernel, ReductionKernel
+from mlc.runtime.executor import CompiledModel
 from workload_cache import graph_of
 
 N, D, FF, H, T, E = 128, 768, 3072, 12, 128, 2  # BERT b1 s128, fp16
@@ -49,3 +52,30 @@ def test_bert_b1_forward_floor():
     mms = [k for k in sched.kernels if isinstance(k, ExternKernel)
            and k.node.op == "aten.mm.default" and k.outputs[0].shape == (N, FF)]
     assert extern_bytes(mms[0]) == (N * D + D * FF + N * FF) * E
+
+
+class _Embedded(torch.nn.Module):
+    def __init__(self):
+        super().__init__()
+        self.table = torch.nn.Embedding(30522, 768)
+        self.up = torch.nn.Linear(768, 3072)
+
+    def forward(self, ids):
+        return torch.relu(self.up(self.table(ids))) * 2.0
+
+
+def test_a_launch_is_priced_by_what_it_moves():
+    """A gather by its rows, not its table; a product and the kernels after it
+    by their operands and outputs, not the product between them. The device
+    estimate that chooses direct launches is built on it."""
+    ids = torch.zeros(4, 32, dtype=torch.int64)
+    sched = build_pipeline(capture(_Embedded().half(), (ids,)), Config(gemm_epilogue=True))
+    (i, (end, _)), = sched.merged.items()
+    assert len(sched.kernels) == 3 and (i, end) == (1, 2)
+    n, w, f = 128, 768, 3072
+    gather, group = 8 * n + 2 * 2 * n * w, 2 * (n * w + w * f + f + n * f)
+    assert launch_bytes(sched.kernels[:1]) == gather
+    assert launch_bytes(sched.kernels[1:]) == group
+    assert launch_bytes(sched.kernels[1:2]) == 2 * (n * w + w * f + n * f)
+    got = CompiledModel._device_estimate([sched.kernels[:1], sched.kernels[1:]])
+    assert got == 3.0 + (gather + group) / 5e6
