@@ -15,10 +15,12 @@ on the replay stream):
   and workgroup size (the cost of dispatching its waves);
 * ``library calls + empty``: the forward with every generated kernel (and the
   native embedding gather) replaced by a one-workgroup empty node, the
-  GEMMs, library or native, real -- what the forward would cost if the fused kernels
-  were free;
+  GEMMs real, library or native, with the pointwise kernels that run in their
+  epilogues -- what the forward would cost if the other fused kernels were
+  free;
 * ``library calls only``: the GEMMs alone;
-* ``forward``: every node real (the executor's graph, re-captured here);
+* ``forward``: every node real (the launches of the executor's pass, captured
+  here);
 * per kernel family (one generated function, every layer's launch of it):
   that family real and every other generated kernel empty. Its excess over
   ``library calls + empty`` is what the family costs above an empty node.
@@ -116,6 +118,7 @@ def decompose_compiled(compiled, inputs, replays: int = 200, families=None, shap
     import torch
 
     from mlc.runtime import native
+    from mlc.runtime.executor import ProductCall
     from mlc.runtime.hip_runtime import Bound
 
     index = compiled.device.index
@@ -137,10 +140,12 @@ def decompose_compiled(compiled, inputs, replays: int = 200, families=None, shap
     dummy = torch.zeros(64, device=device)
     empty_args = struct.pack("<Q", dummy.data_ptr())
 
-    # (kind, bound launch or library call, family symbol) in schedule order
+    # (kind, bound launch or library call, family symbol) in the order of a pass
     entries = []
-    for k, (kind, payload) in zip(compiled.schedule.kernels, compiled._plan):
-        if kind == "kernel":
+    for (k, *more), kind, payload in compiled._launches:
+        if more:  # a product with the pointwise kernels after it
+            entries.append(("lib", ProductCall(rt, payload), None))
+        elif kind == "kernel":
             entries.append(("gen", payload, rt.launch_table[k.name].symbol))
         elif kind == "extern" and k.name in rt.launch_table and getattr(payload, "module", None) is rt:
             entries.append(("gen", payload.bound, rt.launch_table[k.name].symbol))

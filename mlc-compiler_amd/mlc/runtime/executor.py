@@ -322,6 +322,9 @@ class CompiledModel:
         self._buffers = _Buffers(self)
         #: every kernel bound, None where only its group is (``_plan``)
         self._bindings: list | None = None
+        #: what a pass launches: (kernels, kind, payload), a group as one
+        self._launches: list | None = None
+        #: the same with neighbouring native launches in ranges
         self._runs: list | None = None
         #: inputs are read in place and the runs launched one by one
         self._direct = False
@@ -395,26 +398,25 @@ class CompiledModel:
         if len(groups) < len(self.schedule.merged):  # the others' kernels run one by one
             self._buffers.place_unstored()
         bindings: list = [None] * len(self.schedule.kernels)
-        launches, of, i = [], [], 0
+        launches, i = [], 0
         while i < len(bindings):
             k = self.schedule.kernels[i]
             if i in groups:
                 end = self.schedule.merged[i][0]
-                launches.append(("kernel", groups[i]))
-                of.append(self.schedule.kernels[i:end + 1])
+                launches.append((self.schedule.kernels[i:end + 1], "kernel", groups[i]))
                 i = end + 1
                 continue
             bindings[i] = self._bind(k, table)
             if k.name in self._constants:
                 bindings[i][1].run()
-            launches.append(bindings[i])
-            of.append([k])
+            launches.append(([k], *bindings[i]))
             i += 1
-        self._bindings = bindings
+        self._bindings, self._launches = bindings, launches
+        plan = [(kind, payload) for _, kind, payload in launches]
         group = getattr(self._module, "compile_runs", None)
-        self._runs = group(launches) if group is not None else launches
+        self._runs = group(plan) if group is not None else plan
         if (self.cfg.cuda_graphs and self.device.type == "cuda"
-                and hasattr(self._module, "bind_inputs") and self._launch_directly(launches, of)):
+                and hasattr(self._module, "bind_inputs") and self._launch_directly()):
             self._module.bind_inputs(self._runs, {t.data_ptr(): i for i, t in
                                                   enumerate(self._buffers.inputs)})
             mine = {id(t) for t in (*self._buffers.inputs, *self.params.values())}
@@ -423,7 +425,7 @@ class CompiledModel:
                          for t in (*held, *([self._arena] if self._arena is not None else []))]
             self._direct = True
 
-    def _launch_directly(self, launches, of) -> bool:
+    def _launch_directly(self) -> bool:
         """Whether a pass launches its kernels one by one on the caller's own
         inputs rather than replaying a graph behind a copy of them.
 
@@ -441,15 +443,15 @@ class CompiledModel:
             return False
         writes = [v for k in self.schedule.kernels if k.name not in self._constants
                   for v in k.writes()]
-        bound = [c for kind, c in launches if kind == "extern" and isinstance(c, ExternCall)]
-        read = [v for kernels, (_, c) in zip(of, launches) if any(c is x for x in bound)
-                for k in kernels for v in k.reads()]
+        work = [e for e in self._launches if e[1] != "const"]
+        bound = [kernels for kernels, _, c in work if isinstance(c, ExternCall)]
+        read = [v for kernels in bound for k in kernels for v in k.reads()]
         if any(v.buffer.name in names for v in (*self.graph.outputs, *writes, *read)):
             return False
-        count = sum(kind != "const" for kind, _ in launches)
+        count = len(work)
         host = 3.0 * (count - len(bound)) + 9.0 * len(bound)
-        work = [kernels for kernels, (kind, _) in zip(of, launches) if kind != "const"]
-        return count <= MAX_DIRECT and host <= max(24.0, self._device_estimate(work))
+        estimate = self._device_estimate([kernels for kernels, _, _ in work])
+        return count <= MAX_DIRECT and host <= max(24.0, estimate)
 
     @staticmethod
     def _device_estimate(launches) -> float:

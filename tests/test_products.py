@@ -253,3 +253,8 @@ def test_launch_floor_counts_native_products():
     compiled = mlc.compile(torch.nn.Sequential(lin, torch.nn.ReLU()), (x,))
     d = decompose_compiled(compiled, (x,), replays=2, shapes=False, log=lambda line: None)
     assert compiled._module.product_table and d["library"] >= 1 and d["generated"] >= 1
+    # a product that runs the ReLU in its epilogue is one node, as in a pass
+    compiled = mlc.compile(torch.nn.Sequential(lin, torch.nn.ReLU()), (x,), Config(gemm_epilogue=True))
+    d = decompose_compiled(compiled, (x,), replays=2, shapes=False, log=lambda line: None)
+    nodes = {label: n for label, n, _, _ in d["results"]}
+    assert (d["library"], d["generated"], nodes["forward (every node real)"]) == (1, 0, 1)
