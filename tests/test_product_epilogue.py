@@ -278,6 +278,24 @@ def test_results_by_head_size(heads, size):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("b,n,w,h", [(3, 100, 512, 8), (6, 200, 768, 12), (8, 96, 768, 12)])
+def test_merged_projections_with_one_stored_by_columns(b, n, w, h, dtype):
+    """q, k and v out of one launch, one of them transposed by the attention
+    (``store`` and ``store_t`` in one kernel), rows past the last whole tile."""
+    torch.manual_seed(0)
+    model, x = Heads(w, h).to(dtype), torch.randn(b, n, w).to(dtype)
+    want = model.double()(x.double())
+    x, model = x.cuda(), model.to(dtype).cuda()
+    compiled = mlc.compile(model, (x,), ALL)
+    (i, (_, parts)), = compiled.schedule.merged.items()
+    assert "auto store_t =" in emit_group(compiled.schedule.kernels[i], parts)[0]
+    ulp = {torch.float16: 2.0 ** -10, torch.bfloat16: 2.0 ** -7}[dtype]
+    err = (compiled(x).double().cpu() - want).abs().max() / want.abs().max()
+    assert err <= 4 * ulp, err
+
+
+@pytest.mark.gpu
 def test_a_replayed_graph_gives_the_uncaptured_result():
     name, model, args, _ = cases()[2]
     model, args = model.half().cuda(), tuple(a.cuda() for a in args)

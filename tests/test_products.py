@@ -6,8 +6,10 @@ import torch
 
 import mlc
 from mlc.api import build_pipeline
+from mlc.codegen import hip_gemm
 from mlc.codegen.hip_backend import PRELUDE, emit_kernel
-from mlc.codegen.hip_gemm import MERGED_FLOPS, TILED_FLOPS, choose_tile, emit_product, plan_product
+from mlc.codegen.hip_gemm import (LDS_BYTES, MERGED_FLOPS, TILED_FLOPS, TILES, choose_tile, emit_product,
+                                  plan_product)
 from mlc.config import Config
 from mlc.ir.capture import capture
 from mlc.kernels import ExternKernel
@@ -186,6 +188,65 @@ def test_tiled(shape, dtype):
     x, w = _inside(M, K, 8, dtype)._base, _inside(N, K, 8, dtype)._base
     a, b = x[1:-1, 8:-8].double().cpu(), w[1:-1, 8:-8].double().cpu()
     _check(Inner(), (x, w), a @ b.t(), a.abs() @ b.abs().t(), K)
+
+
+class EveryTile(torch.nn.Module):
+    """A product of its own number of rows for each tile, alone and re-laid out
+    per head, the middle third of its columns transposed (the column store)."""
+
+    def __init__(self, K):
+        super().__init__()
+        self.plain = torch.nn.Parameter(torch.randn(525, K))
+        self.heads = torch.nn.Parameter(torch.randn(2304, K))
+
+    def forward(self, x):
+        out = []
+        for i in range(len(TILES)):
+            rows = x[:312 + 16 * i]
+            out.append(torch.mm(rows, self.plain.t()))
+            q, k, v = (t.view(2, -1, 12, 64).transpose(1, 2)
+                       for t in torch.mm(rows, self.heads.t()).chunk(3, -1))
+            out += [q.contiguous(), k.transpose(-2, -1).contiguous(), v.contiguous()]
+        return tuple(out)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,pieces", [(torch.float16, 5), (torch.float16, 1), (torch.bfloat16, 3),
+                                          (torch.float32, 5), (torch.float32, 1)])
+def test_every_tile_at_ragged_sizes(dtype, pieces, monkeypatch):
+    """Every entry of TILES, whatever size would choose it: rows and columns
+    past its last whole tile (312 to 536 rows, 525 columns), k shorter and
+    longer than the ring, stores along rows and along columns."""
+    size, K = dtype.itemsize, 128 // dtype.itemsize * pieces
+
+    def forced(M, N, K, batches, size, math=False):
+        TM, TN, WM, WN, splits = TILES[(M - 312) // 16]
+        WK = max((n for n in splits if pieces % n == 0), default=None)
+        if WK is None:
+            return choose_tile(M, N, K, batches, size, math)
+        stages = next(n for n in (4, 3, 2)
+                      if min(n, pieces // WK) * WK * (TM + TN) * 128 <= LDS_BYTES)
+        return TM, TN, WM, WN, WK, min(stages, max(2, pieces // WK))
+
+    monkeypatch.setattr(hip_gemm, "choose_tile", forced)
+    torch.manual_seed(0)
+    model = EveryTile(K).to(dtype).cuda()
+    x = torch.randn(536, K, device="cuda", dtype=dtype)
+    compiled = mlc.compile(model, (x,), CFG.replace(layout_selection=True))
+    specs = {**compiled._module.product_table, **compiled._module.group_table}
+    assert len(compiled.schedule.merged) == len(TILES) and len(specs) == 2 * len(TILES)
+    got = compiled(x)
+    x, plain, heads = (t.double() for t in (x, model.plain, model.heads))
+    for i in range(len(TILES)):
+        rows = x[:312 + 16 * i]
+        q, k, v = (t.reshape(2, -1, 12, 64).transpose(1, 2) for t in (rows @ heads.t()).chunk(3, -1))
+        wide = [t.reshape(2, -1, 12, 64).transpose(1, 2)
+                for t in (rows.abs() @ heads.abs().t()).chunk(3, -1)]
+        want = [rows @ plain.t(), q, k.transpose(-2, -1), v]
+        sums = [rows.abs() @ plain.abs().t(), wide[0], wide[1].transpose(-2, -1), wide[2]]
+        for g, w, m in zip(got[4 * i:4 * i + 4], want, sums):
+            bound = HALF_ULP[dtype] * w.abs() + (K + 2) * 2.0 ** -24 * m + 2.0 ** -25
+            assert ((g.double() - w).abs() <= bound).all(), (TILES[i], ((g.double() - w).abs() / bound).max())
 
 
 @pytest.mark.gpu
