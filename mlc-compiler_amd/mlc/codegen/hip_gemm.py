@@ -1,10 +1,10 @@
 """Native matrix products for the library calls of a schedule.
 
 ``aten.mm``, ``aten.addmm`` and ``aten.bmm`` stay extern kernels of the
-schedule; where a product is small enough that a library GEMM's fixed cost is
-most of its time, the runtime runs one of the two templates of
-``templates/mlc_gemm.h`` in the library call's place (``plan_product`` decides,
-from sizes, strides and types alone). Both accumulate in fp32 and round once
+schedule; up to the sizes where it was measured to be at least the library's
+speed, the runtime runs one of the two templates of ``templates/mlc_gemm.h`` in
+the library call's place (``plan_product`` decides, from sizes, strides and
+types alone; the lines are ``TILED_FLOPS`` and its neighbours). Both accumulate in fp32 and round once
 to the storage type, as the library does; ``addmm``'s bias is added before that
 rounding.
 
@@ -143,9 +143,10 @@ def choose_tile(M: int, N: int, K: int, batches: int, size: int,
     LDS reads uncovered (4096x768x3072 took 36 us in a layer in 128 x 96 by four
     waves, 27 in 128 x 128 by eight).
 
-    ``math``: an epilogue with a transcendental. No tile then takes more than
-    half of LDS, so that its arithmetic runs beside another tile's products
-    (16384x3072x768 + GELU 104 us in 128 x 192, 111 in 256 x 256).
+    ``math``: an epilogue with a transcendental. With more than one tile per CU
+    none then takes more than half of LDS, so that its arithmetic runs beside
+    another tile's products (16384x3072x768 + GELU 104 us in 128 x 192, 111 in
+    256 x 256); below that a CU has no second tile to run it beside.
 
     In fp32 a k-split of 4 is kept up to 128 rows, where the library sums k in
     as many parts: fewer, longer sums would be further from float64 than it

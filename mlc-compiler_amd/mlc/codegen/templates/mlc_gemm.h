@@ -1,6 +1,6 @@
-// Matrix products on the gfx950 matrix cores, for the sizes where a library
-// GEMM's fixed cost is most of its time: D[m][n] = sum_k A[m][k] B[n][k], fp32
-// accumulation, an epilogue on four consecutive n at a time.
+// Matrix products on the gfx950 matrix cores, for sizes from one row to the
+// tens of GFLOP: D[m][n] = sum_k A[m][k] B[n][k], fp32 accumulation, an epilogue
+// on four consecutive n at a time.
 //
 // A lane's operand fragment is 16 bytes along k: one 16x16x32 step in 16 bits,
 // four 16x16x4 steps in fp32. B's rows are the MFMA's first operand, so a lane

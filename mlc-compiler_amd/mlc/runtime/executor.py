@@ -26,8 +26,8 @@ when the op has an ``.out`` overload taking exactly its arguments plus
 ``out`` (read off the schemas, never by calling it) the result is written
 straight into its buffer; otherwise the op is called and its result copied.
 The HIP runtime may claim an op with a native kernel instead (``NativeCall``:
-the bounds-checked embedding gather; ``ProductCall``: a matrix product small
-enough to beat the library).
+the bounds-checked embedding gather; ``ProductCall``: a matrix product of a size
+where the native kernel is at least the library's speed).
 
 Behaviour kept from the reference runtime (``mlc/runtime/executor.py:41-474``):
 the input checks and their messages, output aliasing, the eager mode, three
@@ -429,14 +429,18 @@ class CompiledModel:
         """Whether a pass launches its kernels one by one on the caller's own
         inputs rather than replaying a graph behind a copy of them.
 
-        A graph costs the host 21 us to launch plus 0.5 a node, and its inputs
-        a copy; a native launch costs 3 us, a library call through torch about
-        9. So one by one wins for a few launches (embeddings b32 s128: 4
-        launches, 42 us as a graph, 18 one by one), and for more while the
-        device has work for longer than the host needs to issue it, where the
-        copy is what is saved. Library calls keep the addresses they were
-        bound with, so none may read an input; no kernel may write one and no
-        output may be one."""
+        A native launch costs the host 3 us, a library call through torch
+        about 9; a graph with its copy of the inputs costs 25 us and 0.5 a
+        node. Chains of tiny kernels, one call after another, one by one /
+        as a graph: 4 launches 16.5 / 26 us, 6 22 / 28, 8 27.5 / 29, 9 30.4 /
+        29.5, 11 36 / 30.5, 15 47 / 37. So eight native launches (24 us) are
+        always made one by one, and more while the device has work for longer
+        than the host needs to issue it, where the copy is what is saved (15
+        launches over 2048 x 2048 fp16: 314 / 323). A call that is waited for
+        by itself gains up to seven launches (35 / 41 us) and pays at eight
+        (53 / 42). Library calls keep the addresses they were bound with, so
+        none may read an input; no kernel may write one and no output may be
+        one."""
         names = {v.buffer.name for v in self.graph.inputs}
         at = {t.data_ptr() for t in self._buffers.inputs if t.numel()}
         if len(at) != len(self._buffers.inputs):
