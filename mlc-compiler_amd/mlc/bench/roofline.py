@@ -18,17 +18,11 @@ from __future__ import annotations
 
 import math
 
-import torch
-
 from ..codegen.index import IndexMap
 from ..kernels import AttentionKernel, ExternKernel, PointwiseKernel, ReductionKernel
 
 #: MI355X published peak HBM3E bandwidth, GB/s
 HBM_PEAK_GBS = 8000.0
-
-
-def _itemsize(dtype: torch.dtype) -> int:
-    return torch.empty((), dtype=dtype).element_size()
 
 
 def distinct_elements(imap: IndexMap) -> int:
@@ -38,15 +32,15 @@ def distinct_elements(imap: IndexMap) -> int:
 def _reads(k) -> dict:
     """Bytes of every distinct operand view of a kernel, by buffer and view."""
     if isinstance(k, ExternKernel):
-        return {(v.buffer.name, v.layout): v.numel * _itemsize(v.dtype) for v in k.inputs}
-    return {(a.value.buffer.name, a.index.render()): distinct_elements(a.index) * _itemsize(a.dtype)
+        return {(v.buffer.name, v.layout): v.numel * v.dtype.itemsize for v in k.inputs}
+    return {(a.value.buffer.name, a.index): distinct_elements(a.index) * a.dtype.itemsize
             for a in k.inputs}
 
 
 def _writes(k) -> dict:
     if isinstance(k, ExternKernel):
-        return {(v.buffer.name, v.layout): v.numel * _itemsize(v.dtype) for v in k.outputs}
-    return {(a.value.buffer.name, a.index.render()): distinct_elements(a.index) * _itemsize(a.dtype)
+        return {(v.buffer.name, v.layout): v.numel * v.dtype.itemsize for v in k.outputs}
+    return {(a.value.buffer.name, a.index): distinct_elements(a.index) * a.dtype.itemsize
             for a in k.outputs}
 
 
@@ -55,7 +49,7 @@ def algorithmic_bytes(k) -> int:
         if k.node.op == "aten.embedding.default":
             out = k.outputs[0]
             ids = k.node.args[1]
-            return 2 * out.numel * _itemsize(out.dtype) + ids.numel * _itemsize(ids.dtype)
+            return 2 * out.numel * out.dtype.itemsize + ids.numel * ids.dtype.itemsize
         raise TypeError(f"no byte model for extern {k.node.op}")
     if not isinstance(k, (PointwiseKernel, ReductionKernel, AttentionKernel)):
         raise TypeError(type(k).__name__)

@@ -441,21 +441,21 @@ class CompiledModel:
         (53 / 42). Library calls keep the addresses they were bound with, so
         none may read an input; no kernel may write one and no output may be
         one."""
+        work = [e for e in self._launches if e[1] != "const"]
+        if len(work) > MAX_DIRECT:
+            return False
         names = {v.buffer.name for v in self.graph.inputs}
         at = {t.data_ptr() for t in self._buffers.inputs if t.numel()}
         if len(at) != len(self._buffers.inputs):
             return False
         writes = [v for k in self.schedule.kernels if k.name not in self._constants
                   for v in k.writes()]
-        work = [e for e in self._launches if e[1] != "const"]
         bound = [kernels for kernels, _, c in work if isinstance(c, ExternCall)]
         read = [v for kernels in bound for k in kernels for v in k.reads()]
         if any(v.buffer.name in names for v in (*self.graph.outputs, *writes, *read)):
             return False
-        count = len(work)
-        host = 3.0 * (count - len(bound)) + 9.0 * len(bound)
-        estimate = self._device_estimate([kernels for kernels, _, _ in work])
-        return count <= MAX_DIRECT and host <= max(24.0, estimate)
+        host = 3.0 * (len(work) - len(bound)) + 9.0 * len(bound)
+        return host <= 24.0 or host <= self._device_estimate([kernels for kernels, _, _ in work])
 
     @staticmethod
     def _device_estimate(launches) -> float:

@@ -135,3 +135,18 @@ def test_the_seams_methods_for_invalid_inputs():
     for name in ("fetch_errors", "pending_error", "clear_errors", "check_errors"):
         assert callable(getattr(HipRuntime, name))
     assert object.__new__(HipRuntime).fetch_errors(0) is None  # nothing to enqueue
+
+
+@pytest.mark.parametrize("launches,asked,direct", [(1, False, True), (8, False, True), (9, True, True),
+                                                   (32, True, True), (33, False, False)])
+def test_the_device_estimate_is_made_only_where_it_decides(launches, asked, direct, monkeypatch):
+    """A first pass pays for it on the host: eight native launches are made
+    one by one whatever it says, more than 32 never are."""
+    a = torch.randn(6, 8)
+    compiled = _compile(Add(), (a, a + 1), _Replaying())
+    asked_for = []
+    monkeypatch.setattr(CompiledModel, "_device_estimate",
+                        staticmethod(lambda work: asked_for.append(len(work)) or 1e9))
+    compiled._launches = compiled._launches * launches
+    assert compiled._launch_directly() == direct
+    assert asked_for == [launches] * asked
