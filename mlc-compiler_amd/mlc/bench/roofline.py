@@ -16,8 +16,6 @@ keeps on chip are not HBM traffic).
 
 from __future__ import annotations
 
-import math
-
 from ..codegen.index import IndexMap
 from ..kernels import AttentionKernel, ExternKernel, PointwiseKernel, ReductionKernel
 
@@ -26,22 +24,34 @@ HBM_PEAK_GBS = 8000.0
 
 
 def distinct_elements(imap: IndexMap) -> int:
-    return math.prod(size for a in imap.axes for size, _, _ in a.terms)
+    n = 1
+    for axis in imap.axes:
+        for size, _, _ in axis.terms:
+            n *= size
+    return n
 
 
-def _reads(k) -> dict:
-    """Bytes of every distinct operand view of a kernel, by buffer and view."""
-    if isinstance(k, ExternKernel):
-        return {(v.buffer.name, v.layout): v.numel * v.dtype.itemsize for v in k.inputs}
-    return {(a.value.buffer.name, a.index): distinct_elements(a.index) * a.dtype.itemsize
-            for a in k.inputs}
-
-
-def _writes(k) -> dict:
-    if isinstance(k, ExternKernel):
-        return {(v.buffer.name, v.layout): v.numel * v.dtype.itemsize for v in k.outputs}
-    return {(a.value.buffer.name, a.index): distinct_elements(a.index) * a.dtype.itemsize
-            for a in k.outputs}
+def _moved(kernels, unstored: str | None = None) -> int:
+    """Bytes of every distinct operand view and every output of ``kernels``
+    but the buffer ``unstored``. Views are compared only where a buffer comes
+    up again: a first pass prices its launches so on the host."""
+    total, seen = 0, {}
+    for k in kernels:
+        if isinstance(k, ExternKernel):
+            reads = [(v.buffer.name, v.layout, v.numel * v.dtype.itemsize) for v in k.inputs]
+            writes = [(v.buffer.name, v.numel * v.dtype.itemsize) for v in k.outputs]
+        else:
+            reads = [(a.value.buffer.name, a.index, distinct_elements(a.index) * a.dtype.itemsize)
+                     for a in k.inputs]
+            writes = [(a.value.buffer.name, distinct_elements(a.index) * a.dtype.itemsize)
+                      for a in k.outputs]
+        for name, view, nbytes in reads:
+            views = seen.setdefault(name, [])
+            if name != unstored and view not in views:
+                views.append(view)
+                total += nbytes
+        total += sum(nbytes for name, nbytes in writes if name != unstored)
+    return total
 
 
 def algorithmic_bytes(k) -> int:
@@ -53,13 +63,13 @@ def algorithmic_bytes(k) -> int:
         raise TypeError(f"no byte model for extern {k.node.op}")
     if not isinstance(k, (PointwiseKernel, ReductionKernel, AttentionKernel)):
         raise TypeError(type(k).__name__)
-    return sum(_reads(k).values()) + sum(_writes(k).values())
+    return _moved([k])
 
 
 def extern_bytes(k: ExternKernel) -> int:
     """Algorithmic bytes of a library call: every distinct operand view read
     once (a GEMM's weights included) plus every output written once."""
-    return sum(_reads(k).values()) + sum(_writes(k).values())
+    return _moved([k])
 
 
 def launch_bytes(kernels) -> int:
@@ -71,11 +81,7 @@ def launch_bytes(kernels) -> int:
         gather = isinstance(first, ExternKernel) and first.node.op == "aten.embedding.default"
         return algorithmic_bytes(first) if gather or not isinstance(first, ExternKernel) \
             else extern_bytes(first)
-    product = first.outputs[0].buffer.name
-    views: dict = {}
-    for k in kernels:
-        views.update(_reads(k) | _writes(k))
-    return sum(n for (name, _), n in views.items() if name != product)
+    return _moved(kernels, first.outputs[0].buffer.name)
 
 
 def forward_bytes(schedule) -> int:
