@@ -10,8 +10,9 @@ registers, as the library stores it, and each kernel's body is evaluated on it
 there. The schedule keeps its kernels (per-kernel profiling times them one by
 one); ``Schedule.merged`` names the groups. The planner keeps every buffer of a
 group alive through all of it and leaves the product out, which is never
-stored: a GPT-2 block's arena is two thirds of what its kernels one by one need
-(b32 s512 fp16: 151 MB for 226).
+stored. What that saves it spends on not writing where the launch before has
+just read (``memory_planning._pack_groups``): a GPT-2 block takes 201 MB at b32
+s512 fp16, its kernels one by one 226.
 """
 
 from __future__ import annotations

@@ -18,6 +18,7 @@ from mlc.kernels import ExternKernel
 from mlc.passes.memory_planning import plan_memory
 from mlc.runtime.native import STATIC_SLAB_BYTES
 from oracle import compile_reference
+from workload_cache import graph_of
 
 ALL = Config(cuda_graphs=False, merge_parallel_gemms=True, gemm_epilogue=True,
              layout_selection=True, fused_attention=True)
@@ -169,6 +170,27 @@ def test_a_group_takes_no_more_memory_than_its_kernels(model, args):
     sched.merged = {}
     assert merged <= plan_memory(sched.graph, sched, ALL).arena_bytes
     assert not _schedule(model, args, ALL.replace(memory_planning=False)).merged
+
+
+@pytest.mark.parametrize("cfg,most", [(Config(gemm_epilogue=True), 0), (ALL, 0),
+                                      (ALL.replace(fused_attention=False), 12)])
+def test_a_launch_does_not_write_where_the_one_before_it_read(cfg, most):
+    """BERT-base b32: within the memory that the kernels one by one need, what
+    a launch read is left alone for one more launch. Without fused attention
+    that memory has no such place for one buffer of a layer."""
+    sched = build_pipeline(graph_of("C4"), cfg)
+    offsets, ranges = sched.plan.offsets, sched.plan.live_ranges.values()
+    end = {j: last for i, (last, _) in sched.merged.items() for j in range(i, last + 1)}
+
+    def share(a, b):
+        x, y = offsets[a.buffer.name], offsets[b.buffer.name]
+        return x < y + b.size and y < x + a.size
+
+    at_once = [(a.buffer.name, b.buffer.name) for a in ranges for b in ranges
+               if a.end < b.start <= end.get(a.end + 1, a.end + 1) and share(a, b)]
+    assert len(at_once) <= most, at_once
+    arena, sched.merged = sched.arena_bytes, {}
+    assert arena <= plan_memory(sched.graph, sched, cfg).arena_bytes
 
 
 def test_the_static_arena_holds_what_it_held():
