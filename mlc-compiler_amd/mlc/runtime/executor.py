@@ -455,7 +455,14 @@ class CompiledModel:
         if any(v.buffer.name in names for v in (*self.graph.outputs, *writes, *read)):
             return False
         host = 3.0 * (len(work) - len(bound)) + 9.0 * len(bound)
-        return host <= 24.0 or host <= self._device_estimate([kernels for kernels, _, _ in work])
+        if host <= 24.0:
+            return True
+        launches = [kernels for kernels, _, _ in work]
+        # the whole of every buffer is more than moves, and quickly added up
+        most = sum(v.buffer.nbytes for kernels in launches for k in kernels
+                   for v in (*k.reads(), *k.writes()))
+        return (host <= 1.5 * len(launches) + most / 5e6
+                and host <= self._device_estimate(launches))
 
     @staticmethod
     def _device_estimate(launches) -> float:

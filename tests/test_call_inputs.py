@@ -137,12 +137,14 @@ def test_the_seams_methods_for_invalid_inputs():
     assert object.__new__(HipRuntime).fetch_errors(0) is None  # nothing to enqueue
 
 
-@pytest.mark.parametrize("launches,asked,direct", [(1, False, True), (8, False, True), (9, True, True),
-                                                   (32, True, True), (33, False, False)])
-def test_the_device_estimate_is_made_only_where_it_decides(launches, asked, direct, monkeypatch):
+@pytest.mark.parametrize("launches,rows,asked,direct", [
+    (1, 6, False, True), (8, 6, False, True), (9, 6, False, False), (9, 1 << 20, True, True),
+    (32, 1 << 20, True, True), (33, 1 << 20, False, False)])
+def test_the_device_estimate_is_made_only_where_it_decides(launches, rows, asked, direct, monkeypatch):
     """A first pass pays for it on the host: eight native launches are made
-    one by one whatever it says, more than 32 never are."""
-    a = torch.randn(6, 8)
+    one by one whatever it says, more than 32 never are, and nine not where
+    the buffers themselves are too small to keep the device busy."""
+    a = torch.zeros(rows, 8)
     compiled = _compile(Add(), (a, a + 1), _Replaying())
     asked_for = []
     monkeypatch.setattr(CompiledModel, "_device_estimate",
