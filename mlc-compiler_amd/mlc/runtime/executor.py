@@ -287,13 +287,15 @@ class _Buffers:
 # the model
 # --------------------------------------------------------------------------
 
-def _plain(t: torch.Tensor, own: torch.Tensor) -> bool:
-    """Whether a kernel may read the caller's ``t`` at its address in the place
-    of the input buffer ``own``: the same bytes, on 16 of them, and in memory
-    at all (torch's efficient zero tensors are not)."""
-    return (type(t) is torch.Tensor and t.dtype == own.dtype and t.device == own.device
-            and t.is_contiguous() and not t.is_neg() and not t._is_zerotensor()
-            and t.data_ptr() % 16 == 0)
+def _address(t: torch.Tensor, own: torch.Tensor) -> int:
+    """Where a kernel may read the caller's ``t`` in the place of the input
+    buffer ``own``, or 0: the same bytes, on 16 of them, and in memory at all
+    (torch's efficient zero tensors have a null address)."""
+    if (type(t) is torch.Tensor and t.dtype == own.dtype and t.device == own.device
+            and t.is_contiguous() and not t.is_neg()):
+        at = t.data_ptr()
+        return 0 if at % 16 else at
+    return 0
 
 
 def _alloc_count(device) -> int:
@@ -481,11 +483,9 @@ class CompiledModel:
         (an output fed back)."""
         out = []
         for t, own in zip(inputs, self._buffers.inputs):
-            if not _plain(t, own):
-                return None
-            p = t.data_ptr()
-            end = p + own.numel() * own.element_size()
-            if any(p < hi and lo < end for lo, hi in self._own):
+            p = _address(t, own)
+            end = p + own.nbytes
+            if not p or any(p < hi and lo < end for lo, hi in self._own):
                 return None
             out.append(p)
         return out
@@ -515,8 +515,9 @@ class CompiledModel:
                       for t, own in zip(inputs, self._buffers.inputs)]
         copies = []
         for t, own in zip(inputs, self._buffers.inputs):
-            if len(copies) < self._module.MAX_COPIES and _plain(t, own):
-                copies.append((own.data_ptr(), t.data_ptr(), own.numel() * own.element_size()))
+            at = _address(t, own) if len(copies) < self._module.MAX_COPIES else 0
+            if at:
+                copies.append((own.data_ptr(), at, own.nbytes))
             else:
                 own.copy_(t.reshape(-1), non_blocking=True)
         self._module.graph_call(copies, stream.cuda_stream)
